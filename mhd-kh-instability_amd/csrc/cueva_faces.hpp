@@ -8,6 +8,7 @@
 #include <stddef.h>
 
 #include <type_traits>
+#include <utility>
 
 #include "cueva_common.hpp"
 #include "cueva_update.hpp"
@@ -31,6 +32,13 @@
 
 namespace cueva {
 
+// Stencils loaded ahead of the one being reconstructed.  Step times at
+// 2048x4096, HLLC + MP5, with 0 / 1 / 2 / 3: FP64 7.28 / 6.23 / 5.87 / 5.82 ms
+// (MP9 at 768x1536 3.34 / 2.97 / 2.94 / 2.93), mixed 4.57 / 4.32 / 4.32 / 4.40,
+// mixed HLLE + MP7 at 1024x2048 1.46 / 1.39 / 1.42 / 1.50: FP64 has the
+// registers for two (2 waves per SIMD), FP32 at 128 has them for one.
+template <typename T> constexpr int face_ahead() { return sizeof(T) == 8 ? 2 : 1; }
+
 // launch grid of k_faces over the face pairs [-1,imax] x [-1,jmax]
 inline dim3 faces_grid(const Geom& g, dim3 blk) {
   const unsigned tx = (unsigned)((g.imax + 2 + blk.x - 1) / blk.x), ty = (unsigned)((g.jmax + 2 + blk.y - 1) / blk.y);
@@ -46,41 +54,94 @@ inline dim3 faces_grid(const Geom& g, dim3 blk) {
 // face between (i,j),(i+1,j) and the y face between (i,j),(i,j+1), for
 // i in [-1,imax], j in [-1,jmax] (16_*_flow_mpx.f95 face loops)
 // ---------------------------------------------------------------------------
-template <int ORD, typename T>
-__device__ inline void face_rec(const double* __restrict__ a, int64_t c, int64_t st, T& L, T& R) {
-  constexpr int K = MPc<ORD>::K;
-  T v[2 * K + 2];
-#pragma unroll
-  for (int t = 0; t < 2 * K + 2; t++) v[t] = (T)a[c + (int64_t)(t - K) * st];
-  mp_face<ORD>(v, L, R);
+// The cell a face solve stands at, split for the addressing of a wavefront:
+// its 64 lanes share the row, so a plane's row address is formed on scalar
+// registers and each lane adds only its 32-bit byte offset within the row
+// (global loads take a scalar base, a 32-bit lane offset and a constant).
+struct Cell {
+  uint32_t vo;   // byte offset of column i in its row
+  int64_t ro;    // first element of row j (the same for every lane)
+  int pitch;
+};
+__device__ inline Cell cell_of(const Geom& g, int i, int j) {
+  return {(uint32_t)(i + 8) * 8u, (int64_t)(__builtin_amdgcn_readfirstlane(j) + GH) * g.pitch, g.pitch};
 }
-template <int ORD, typename T>
-__device__ inline void face_rec_pos(const double* __restrict__ a, int64_t c, int64_t st, T& L, T& R) {
-  constexpr int K = MPc<ORD>::K;
-  T v[2 * K + 2];
-#pragma unroll
-  for (int t = 0; t < 2 * K + 2; t++) v[t] = (T)a[c + (int64_t)(t - K) * st];
-  mp_face_pos<ORD>(v, L, R);
+// element (i + DI, j + dj)
+template <int DI = 0> __device__ inline double at_cell(const double* __restrict__ a, const Cell& c, int dj = 0) {
+  const char* row = (const char*)(a + (c.ro + (int64_t)dj * c.pitch));
+  return *(const double*)(row + c.vo + DI * 8);
 }
 
-// reconstruct every non-kinematic quantity of one face (slots 1-20, 26/27/63)
-template <int ORD, int DIR, typename T>
-__device__ inline void face_fields(const Planes& P, int64_t c, int64_t st, Side<T>& L, Side<T>& R) {
-  face_rec<ORD>(P.s[S_PSI], c, st, L.psi, R.psi);
-  face_rec<ORD>(P.s[S_PHI], c, st, L.phi, R.phi);
-  face_rec<ORD>(P.s[S_EX], c, st, L.ex, R.ex);
-  face_rec<ORD>(P.s[S_EY], c, st, L.ey, R.ey);
-  face_rec<ORD>(P.s[S_EZ], c, st, L.ez, R.ez);
-  face_rec<ORD>(P.s[S_BX], c, st, L.bx, R.bx);
-  face_rec<ORD>(P.s[S_BY], c, st, L.by, R.by);
-  face_rec<ORD>(P.s[S_BZ], c, st, L.bz, R.bz);
-  face_rec<ORD>(P.s[S_Q], c, st, L.q, R.q);
-  face_rec<ORD>(P.s[S_D], c, st, L.d, R.d);
-  face_rec<ORD>(P.s[S_TAU], c, st, L.tau, R.tau);
-  face_rec<ORD>(P.s[S_SX], c, st, L.sx, R.sx);
-  face_rec<ORD>(P.s[S_SY], c, st, L.sy, R.sy);
-  face_rec<ORD>(P.s[S_SZ], c, st, L.sz, R.sz);
-  face_rec<ORD>(P.s[DIR == 0 ? S_JX : S_JY], c, st, L.jn, R.jn);
+// the 2K+2 values of one quantity across the face, as loaded (FP64)
+template <int ORD> struct Sten { double v[2 * MPc<ORD>::K + 2]; };
+template <int ORD, int DIR, int... T>
+__device__ inline void sten_load(const double* __restrict__ a, const Cell& c, Sten<ORD>& s,
+                                 std::integer_sequence<int, T...>) {
+  constexpr int K = MPc<ORD>::K;
+  ((s.v[T] = DIR == 0 ? at_cell<DIR == 0 ? T - K : 0>(a, c) : at_cell(a, c, T - K)), ...);
+}
+
+// quantities reconstructed at a face, in the order they are taken: the
+// kinematics first (the fallbacks couple the two faces of a pair)
+enum { F_VX, F_VY, F_VZ, F_P, F_RHO, F_PSI, F_PHI, F_EX, F_EY, F_EZ, F_BX, F_BY, F_BZ, F_Q, F_D, F_TAU, F_SX, F_SY,
+       F_SZ, F_JN, F_NQ };
+template <int F, int DIR, bool STAGE_KIN> __device__ inline const double* face_plane(const Planes& P) {
+  if constexpr (F <= F_RHO) {
+    constexpr int q = F == F_VX ? K_VX : F == F_VY ? K_VY : F == F_VZ ? K_VZ : F == F_P ? K_P : K_RHO;
+    return kin_plane<STAGE_KIN>(P, q);
+  } else {
+    constexpr int s[15] = {S_PSI, S_PHI, S_EX, S_EY, S_EZ, S_BX, S_BY, S_BZ, S_Q, S_D, S_TAU, S_SX, S_SY, S_SZ,
+                           DIR == 0 ? S_JX : S_JY};
+    constexpr int k = s[F - F_PSI];
+    return P.s[k];
+  }
+}
+template <int F, typename T> __device__ inline T& face_slot(Side<T>& o) {
+  constexpr T Side<T>::*m[F_NQ] = {&Side<T>::vx, &Side<T>::vy, &Side<T>::vz, &Side<T>::p, &Side<T>::rho,
+                                   &Side<T>::psi, &Side<T>::phi, &Side<T>::ex, &Side<T>::ey, &Side<T>::ez,
+                                   &Side<T>::bx, &Side<T>::by, &Side<T>::bz, &Side<T>::q, &Side<T>::d,
+                                   &Side<T>::tau, &Side<T>::sx, &Side<T>::sy, &Side<T>::sz, &Side<T>::jn};
+  return o.*m[F];
+}
+
+template <int ORD, int F, int DIR, bool STAGE_KIN>
+__device__ inline void face_load(const Planes& P, const Cell& c, Sten<ORD>& s) {
+  sten_load<ORD, DIR>(face_plane<F, DIR, STAGE_KIN>(P), c, s,
+                      std::make_integer_sequence<int, 2 * MPc<ORD>::K + 2>());
+}
+template <int ORD, int F, typename T>
+__device__ inline void face_take(const Sten<ORD>& s, Side<T>& L, Side<T>& R) {
+  constexpr int N = 2 * MPc<ORD>::K + 2;
+  T v[N];
+#pragma unroll
+  for (int t = 0; t < N; t++) v[t] = (T)s.v[t];
+  if constexpr (F == F_P || F == F_RHO) mp_face_pos<ORD>(v, face_slot<F>(L), face_slot<F>(R));
+  else mp_face<ORD>(v, face_slot<F>(L), face_slot<F>(R));
+}
+
+// Reconstruct quantities F0 + S... of one face.  The stencils of the next
+// quantities are loaded before the current one is reconstructed: the
+// limiter's wavefront-wide branch keeps the compiler from moving loads across
+// it, and without this every quantity waited for its own loads.
+template <int ORD, int F0, int DIR, bool STAGE_KIN, typename T, int... S>
+__device__ inline void face_fields_seq(const Planes& P, const Cell& c, Side<T>& L, Side<T>& R,
+                                       std::integer_sequence<int, S...>) {
+  constexpr int N = sizeof...(S), AH = face_ahead<T>();
+  Sten<ORD> b[AH + 1];
+  auto pre = [&](auto t) {
+    if constexpr (t() < AH && t() < N) face_load<ORD, F0 + t(), DIR, STAGE_KIN>(P, c, b[t()]);
+  };
+  auto one = [&](auto t) {
+    if constexpr (t() + AH < N)
+      face_load<ORD, F0 + t() + AH, DIR, STAGE_KIN>(P, c, b[(t() + AH) % (AH + 1)]);
+    face_take<ORD, F0 + t()>(b[t() % (AH + 1)], L, R);
+  };
+  (pre(std::integral_constant<int, S>()), ...);
+  (one(std::integral_constant<int, S>()), ...);
+}
+template <int ORD, int F0, int F1, int DIR, bool STAGE_KIN, typename T>
+__device__ inline void face_fields(const Planes& P, const Cell& c, Side<T>& L, Side<T>& R) {
+  face_fields_seq<ORD, F0, DIR, STAGE_KIN>(P, c, L, R, std::make_integer_sequence<int, F1 - F0>());
 }
 
 // ---------------------------------------------------------------------------
@@ -423,16 +484,9 @@ __device__ __forceinline__ void face_pair(const Geom& g, const Planes& P, const 
   }
   Side<T> xl, xr, yl, yr;
   // kinematics of both faces first: the fallbacks couple them
-  face_rec<ORD>(kin_plane<STAGE_KIN>(P, K_VX), c, sx, xl.vx, xr.vx);
-  face_rec<ORD>(kin_plane<STAGE_KIN>(P, K_VY), c, sx, xl.vy, xr.vy);
-  face_rec<ORD>(kin_plane<STAGE_KIN>(P, K_VZ), c, sx, xl.vz, xr.vz);
-  face_rec<ORD>(kin_plane<STAGE_KIN>(P, K_VX), c, sy, yl.vx, yr.vx);
-  face_rec<ORD>(kin_plane<STAGE_KIN>(P, K_VY), c, sy, yl.vy, yr.vy);
-  face_rec<ORD>(kin_plane<STAGE_KIN>(P, K_VZ), c, sy, yl.vz, yr.vz);
-  face_rec_pos<ORD>(kin_plane<STAGE_KIN>(P, K_P), c, sx, xl.p, xr.p);
-  face_rec_pos<ORD>(kin_plane<STAGE_KIN>(P, K_RHO), c, sx, xl.rho, xr.rho);
-  face_rec_pos<ORD>(kin_plane<STAGE_KIN>(P, K_P), c, sy, yl.p, yr.p);
-  face_rec_pos<ORD>(kin_plane<STAGE_KIN>(P, K_RHO), c, sy, yl.rho, yr.rho);
+  const Cell cc = cell_of(g, i, j);
+  face_fields<ORD, F_VX, F_PSI, 0, STAGE_KIN>(P, cc, xl, xr);
+  face_fields<ORD, F_VX, F_PSI, 1, STAGE_KIN>(P, cc, yl, yr);
   // superluminal fallback, 16_hll_flow_mpx.f95:1392-1461 (same in hllc;
   // hlle only prints, 16_hlle_flow_mpx.f95:2270-2300)
   if (SOLVER != 6) {
@@ -460,14 +514,14 @@ __device__ __forceinline__ void face_pair(const Geom& g, const Planes& P, const 
   // is the y face's (E x B)_y; that of the y solve is the x solve's last iterate
   T seed_x = T(0), seed_y = T(0);
   if (SOLVER == 6 && S.hllc_seed_ref) {
-    face_rec<ORD>(P.s[S_EX], c, sy, yl.ex, yr.ex);
-    face_rec<ORD>(P.s[S_EZ], c, sy, yl.ez, yr.ez);
-    face_rec<ORD>(P.s[S_BX], c, sy, yl.bx, yr.bx);
-    face_rec<ORD>(P.s[S_BZ], c, sy, yl.bz, yr.bz);
+    face_fields<ORD, F_EX, F_EX + 1, 1, STAGE_KIN>(P, cc, yl, yr);
+    face_fields<ORD, F_EZ, F_EZ + 1, 1, STAGE_KIN>(P, cc, yl, yr);
+    face_fields<ORD, F_BX, F_BX + 1, 1, STAGE_KIN>(P, cc, yl, yr);
+    face_fields<ORD, F_BZ, F_BZ + 1, 1, STAGE_KIN>(P, cc, yl, yr);
     seed_x = hlle_y_ery(yl, yr);
   }
   auto xface = [&]() {
-    face_fields<ORD, 0>(P, c, sx, xl, xr);
+    face_fields<ORD, F_PSI, F_NQ, 0, STAGE_KIN>(P, cc, xl, xr);
     side_physics<0, HW>((T)S.gamma, xl);
     side_physics<0, HW>((T)S.gamma, xr);
     T f[FX_N];
@@ -483,7 +537,7 @@ __device__ __forceinline__ void face_pair(const Geom& g, const Planes& P, const 
     put_x(f);
   };
   auto yface = [&]() {
-    face_fields<ORD, 1>(P, c, sy, yl, yr);
+    face_fields<ORD, F_PSI, F_NQ, 1, STAGE_KIN>(P, cc, yl, yr);
     side_physics<1, HW>((T)S.gamma, yl);
     side_physics<1, HW>((T)S.gamma, yr);
     T f[FY_N];
