@@ -32,12 +32,11 @@
 
 namespace cueva {
 
-// Stencils loaded ahead of the one being reconstructed.  Step times at
-// 2048x4096, HLLC + MP5, with 0 / 1 / 2 / 3: FP64 7.28 / 6.23 / 5.87 / 5.82 ms
-// (MP9 at 768x1536 3.34 / 2.97 / 2.94 / 2.93), mixed 4.57 / 4.32 / 4.32 / 4.40,
-// mixed HLLE + MP7 at 1024x2048 1.46 / 1.39 / 1.42 / 1.50: FP64 has the
-// registers for two (2 waves per SIMD), FP32 at 128 has them for one.
-template <typename T> constexpr int face_ahead() { return sizeof(T) == 8 ? 2 : 1; }
+// Stencils loaded ahead of the one being reconstructed.  FP64 (2 waves per
+// SIMD, HLLC + MP5 at 2048x4096, step with 0 / 1 / 2 / 3): 6.6 / 5.53 / 5.19 /
+// 5.12 ms.  FP32 takes two at 3 waves per SIMD (4.16 ms; one at 3 waves 4.25,
+// one at 4 waves, which spill, 4.46, three at 2 waves 4.15).
+template <typename T> constexpr int face_ahead() { return sizeof(T) == 8 ? 3 : 2; }
 
 // launch grid of k_faces over the face pairs [-1,imax] x [-1,jmax]
 inline dim3 faces_grid(const Geom& g, dim3 blk) {
@@ -658,14 +657,14 @@ static_assert(offsetof(MarchArgs, P) == 0, "argument block layout");
 //     more than 256 and ran 1 wave per SIMD unbounded: bounded, HLL spills
 //     2-12 VGPRs and runs 36 % faster, HLLE (one y-row buffer, below) 36 %,
 //     Lax-Friedrichs 32 %, the MCL solvers (63-114 spilled) 17-20 %;
-//   FP32: 4 for HLLC (2 VGPRs spill) and HLLE (8-22 spill; 3 %), 3 for the
-//     others: the MCL solvers' 178-192 VGPRs ran 2 waves per SIMD unbounded
-//     and 9-19 % slower; HLL and Lax-Friedrichs fit 3 unbounded, and at 4
-//     HLL spills 25-56 VGPRs and ran 19 % slower, Lax-Friedrichs 29 and 6 %.
+//   FP32: 3.  With the stencils loaded ahead, 4 waves (128 VGPRs) spill
+//     22-37 VGPRs under HLLC and ran 7 % slower (HLLE 13 %), 2 the same; the
+//     MCL solvers' 178-192 VGPRs ran 2 waves per SIMD unbounded and 9-19 %
+//     slower.
 template <typename T, int SOLVER>
 constexpr int march_min_waves() {
   if constexpr (sizeof(T) == 8) return CUEVA_MARCH_F64_WAVES > 0 ? CUEVA_MARCH_F64_WAVES : 2;
-  else return CUEVA_MARCH_F32_WAVES > 0 ? CUEVA_MARCH_F32_WAVES : (SOLVER == 7 || SOLVER == 6 ? 4 : 3);
+  else return CUEVA_MARCH_F32_WAVES > 0 ? CUEVA_MARCH_F32_WAVES : 3;
 }
 
 // y-face row buffers: 2 (one barrier per tile step), or 1 for HLLE (a second
@@ -775,11 +774,11 @@ k_faces_march(MarchArgs args) {
 #pragma unroll
         for (int t = 0; t < R_N; t++) P.rhs[l][t][k] = r.r[t];
         // the next stage's state of this point (pointwise in U^n and the
-        // stage right-hand sides, the last of which was just stored)
+        // stage right-hand sides, the last of which is still in registers)
         double sv[S_N];
         stage_point(P, S, l + 1, k, false, P.p[P_VX][k], P.p[P_VY][k], P.p[P_VZ][k], P.p[P_EX][k], P.p[P_EY][k],
                     P.p[P_EZ][k], P.p[P_BX][k], P.p[P_BY][k], P.p[P_BZ][k], P.p[P_RHO][k], P.p[P_P][k],
-                    P.p[P_PSI][k], P.p[P_PHI][k], P.p[P_Q][k], sv);
+                    P.p[P_PSI][k], P.p[P_PHI][k], P.p[P_Q][k], sv, &r);
         store_stage(P.sn, k, sv);
       } else {
         double nu[A_N];
