@@ -55,7 +55,7 @@ struct cueva_ctx {
   int has_mlp;
   int rec_order;
   int march;         // fused step uses the marching face kernel (default; CUEVA_MARCH=0: face planes)
-  int march_rounds;  // resident-block rounds a marching launch is cut into (CUEVA_MARCH_ROUNDS)
+  int march_rounds;  // resident-block rounds a marching launch is cut into when set (CUEVA_MARCH_ROUNDS)
   int march_xcd;     // marching blocks in XCD-aware tile order (CUEVA_MARCH_XCD, default on)
   int march_rows;    // rows per segment when set (CUEVA_MARCH_SEG; rounded up to 4m - 1)
   int c2p_in_march;  // Cardano recovery inside the last marching launch (CUEVA_C2P_IN_MARCH)
@@ -277,12 +277,8 @@ extern "C" int cueva_create(const cueva_params* p, cueva_ctx** out) {
   {
     const char* e = getenv("CUEVA_MARCH");
     c->march = e ? atoi(e) != 0 : 1;
-    // resident-block rounds a marching launch is cut into: measured best at
-    // 4 for the FP64 kernels (2 blocks per CU; 1.5-3.6 % faster than 2 at
-    // 2048x4096 and 4096x8192) and 2 for the FP32 ones (4 blocks per CU):
-    // about 2000 blocks of ~67-row segments at 2048x4096 either way
     e = getenv("CUEVA_MARCH_ROUNDS");
-    c->march_rounds = e && atoi(e) > 0 ? atoi(e) : (p->precision == CUEVA_MIXED ? 2 : 4);
+    c->march_rounds = e && atoi(e) > 0 ? atoi(e) : 0;
     // the hardware deals workgroups to the 8 XCDs round robin; in the XCD-aware
     // order each XCD marches a contiguous band of tiles, whose neighbours
     // share halo columns and rows in its L2: 19-25 % fewer bytes fetched and
@@ -880,9 +876,20 @@ static void recover_to_scratch(cueva_ctx* c) {
   for (int q = 0; q < 5; q++) c->P.pn[q] = c->P.fx[q];
 }
 
-// Rows per segment of a marching launch: enough segments that the blocks
-// fill the resident slots of every CU march_rounds times, seg = MW m - 1 (the
-// segment's face rows, seg + 1, fill whole tile steps of MW rows).
+// Rows per segment of a marching launch: seg = MW m - 1, so that the
+// segment's face rows, seg + 1, fill m whole tile steps of MW rows.  m is the
+// one with the smallest of
+//   rounds m        tile steps that a resident slot runs in turn, rounds =
+//                   blocks / slots rounded up (a last, nearly empty round
+//                   costs as much as a full one),
+//   + blocks m / slots    the work with its redundant first face rows, shared
+//                   by the slots of a CU,
+//   + m / 10        the blocks of a single long round end apart (the limiters
+//                   run in some strips only).
+// Step times it goes by, FP64 HLLC at 512 slots, m (rounds): 509x1021 5 (1)
+// 436 us, 1 (6) 477, 3 (2) 487, 2 (3) 507; 2048x4096 17 (4) 5.12 ms, 34 (2)
+// 5.20, 23 (3) 5.21, 12 (6) 5.26, 69 (1) 5.34; MP9 768x1536 11 (1) 2.29 ms,
+// 2 (6) 2.31, 3 (4) 2.31, 6 (2) 2.37.  The FP32 forms move within 2 %.
 static int march_seg(cueva_ctx* c, bool fin, bool c2p) {
   int& seg = c->march_seg[fin ? (c2p ? 2 : 1) : 0];
   if (seg) return seg;
@@ -898,10 +905,23 @@ static int march_seg(cueva_ctx* c, bool fin, bool c2p) {
     return 0;
   const int64_t slots = (int64_t)(per_cu > 0 ? per_cu : 1) * (cus > 0 ? cus : 1);
   const int strips = march_strips(c->g), rows = c->g.jmax + 1;
-  int64_t want = slots * c->march_rounds / strips;
-  if (want < 1) want = 1;
-  const int64_t per = (rows + want - 1) / want;
-  const int64_t m = (per + 1 + mw - 1) / mw;
+  int64_t m = 1;
+  if (c->march_rounds > 0) {
+    int64_t want = slots * c->march_rounds / strips;
+    if (want < 1) want = 1;
+    const int64_t per = (rows + want - 1) / want;
+    m = (per + 1 + mw - 1) / mw;
+  } else {
+    int64_t best = INT64_MAX;
+    for (int64_t t = 1; t <= (rows + 1 + mw - 1) / mw; t++) {
+      const int64_t blocks = strips * ((rows + mw * t - 2) / (mw * t - 1)), rounds = (blocks + slots - 1) / slots;
+      const int64_t cost = 10 * (rounds * t * slots + blocks * t) + t * slots;
+      if (cost < best) {
+        best = cost;
+        m = t;
+      }
+    }
+  }
   seg = (int)(mw * m - 1);
   return seg;
 }
