@@ -475,7 +475,9 @@ static int fill_ghosts(cueva_ctx* c, double* const* planes, int n, int nzero = 0
     pl.nzero = start + pl.n == n ? nzero : 0;
     for (int k = 0; k < pl.n; k++) pl.a[k] = planes[start + k];
     int64_t cnt = ghost_count(c->g);
-    LAUNCH(K_GHOSTS, k_fill_ghosts, dim3((unsigned)((cnt + 255) / 256)), dim3(256), c->g, pl, sr);
+    LAUNCH(K_GHOSTS, k_fill_ghosts,
+           dim3((unsigned)((cnt + 255) / 256), (unsigned)((pl.n + GHOST_PLANES - 1) / GHOST_PLANES)), dim3(256), c->g, pl,
+           sr);
     if (launch_ok()) return CUEVA_E_HIP;
   }
   return CUEVA_OK;
