@@ -6,9 +6,14 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <sched.h>
+
 #include <algorithm>
+#include <atomic>
+#include <exception>
 #include <mutex>
 #include <new>
+#include <thread>
 #include <vector>
 
 #include "cueva.h"
@@ -41,6 +46,16 @@ struct LaunchRecord {
 constexpr size_t MAX_LAUNCH_RECORDS = 16384;
 constexpr int FIX_CAP = 1 << 16;  // fix-up records kept per kind between reads
 
+// pinned host buffers of the transfers to and from host arrays (copy_planes)
+constexpr size_t IO_CHUNK = (size_t)4 << 20;  // bytes of one buffer at most
+constexpr int IO_MAX_THREADS = 8;
+
+struct PinnedPair {
+  double* buf[2];
+  hipEvent_t done[2];
+  size_t bytes;  // of each
+};
+
 struct cueva_ctx {
   cueva_params prm;
   Geom g;
@@ -67,6 +82,7 @@ struct cueva_ctx {
   std::vector<LaunchRecord>* launches;
   int err;              // first failure (sticky until the next upload of primitives)
   int32_t err_where[4]; // its step, stage, i, j
+  PinnedPair io[IO_MAX_THREADS];  // host transfers: the buffers of each thread, made when first needed
   // kernel timing (cueva_set_profiling)
   int prof;
   int nev, capev;
@@ -385,6 +401,8 @@ extern "C" int cueva_create(const cueva_params* p, cueva_ctx** out) {
   return CUEVA_OK;
 }
 
+static void io_release(PinnedPair& p);
+
 extern "C" int cueva_destroy(cueva_ctx* c) {
   if (!c) return CUEVA_E_ARG;
   hipStreamSynchronize(c->stream);
@@ -392,6 +410,7 @@ extern "C" int cueva_destroy(cueva_ctx* c) {
   for (int k = 0; k < 2 * c->capev; k++) hipEventDestroy(c->ev[k]);
   free(c->ev);
   free(c->evcls);
+  for (PinnedPair& p : c->io) io_release(p);
   hipFree(c->dst);
   hipFree(c->base);
   hipStreamDestroy(c->stream);
@@ -414,25 +433,173 @@ extern "C" int cueva_device_bytes(const cueva_ctx* c, int64_t* bytes) {
 // ---------------------------------------------------------------------------
 // host <-> device
 // ---------------------------------------------------------------------------
-static int copy_planes_h2d(cueva_ctx* c, double* const* dst, int n, const double* host) {
+// Host arrays hold the planes one after the other with imax+13 doubles a row;
+// a device plane has the context's pitch.  A strided copy of pageable memory
+// goes row by row (5 to 10 us a row: 0.55 s for the 57526 rows up at
+// 2048x4096, 1.7 GB/s, and 12 ms at 32x64), so the rows go through pinned
+// buffers instead: a host thread copies a run of rows into one (or out of
+// one) and a kernel places them in the planes (or gathers them), reading and
+// writing the pinned memory over the link itself, with no device staging.
+// Each thread keeps two buffers, so that its memory copy and the kernel of its
+// other buffer overlap.  Large transfers take several threads (one copies
+// 12 GB/s into fresh pages, 30 into warm ones; the link carries 57).  Up / down
+// now 19.6 / 19.3 ms (48 GB/s) at 2048x4096, 0.06 / 0.04 ms at 32x64.
+static void io_release(PinnedPair& p) {
+  for (int k = 0; k < 2; k++) {
+    if (p.buf[k]) hipHostFree(p.buf[k]);
+    if (p.done[k]) hipEventDestroy(p.done[k]);
+    p.buf[k] = nullptr;
+    p.done[k] = nullptr;
+  }
+  p.bytes = 0;
+}
+
+// buffers of at least `bytes` each; false if they cannot be had
+static bool io_reserve(PinnedPair& p, size_t bytes) {
+  if (p.bytes >= bytes) return true;
+  io_release(p);
+  for (int k = 0; k < 2; k++) {
+    void* b = nullptr;
+    if (hipHostMalloc(&b, bytes, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess) {
+      (void)hipGetLastError();
+      io_release(p);
+      return false;
+    }
+    p.buf[k] = (double*)b;
+    if (hipEventCreateWithFlags(&p.done[k], hipEventDisableTiming) != hipSuccess) {
+      p.done[k] = nullptr;
+      io_release(p);
+      return false;
+    }
+  }
+  p.bytes = bytes;
+  return true;
+}
+
+// one transfer: n planes of hh rows of w doubles, in runs of `run` rows that
+// the threads take in turn
+struct IoJob {
+  cueva_ctx* c;
+  PlaneList pl;
+  double* host;
+  int up, w, hh, run, runs, dev;
+  std::atomic<int> next;
+  std::atomic<int> err;
+};
+
+static bool io_launch(const IoJob& j, double* buf, int r0, int rows) {
+  const dim3 grid((unsigned)((j.w + 255) / 256), (unsigned)((rows + 3) / 4)), blk(64, 4);
+  if (j.up)
+    hipLaunchKernelGGL(k_rows_to_planes, grid, blk, 0, j.c->stream, (const double*)buf, j.pl, j.w, j.hh, j.c->g.pitch, r0, rows);
+  else
+    hipLaunchKernelGGL(k_planes_to_rows, grid, blk, 0, j.c->stream, buf, j.pl, j.w, j.hh, j.c->g.pitch, r0, rows);
+  return hipGetLastError() == hipSuccess;
+}
+
+// one thread's share: runs are taken from the job until none is left
+static void io_work(IoJob& j, PinnedPair& p) {
+  const int total = j.pl.n * j.hh;
+  int r0[2] = {-1, -1}, rows[2] = {0, 0}, k = 0;
+  bool ok = true;
+  auto finish = [&](int b) {  // the buffer's kernel has ended; downloads copy its rows out
+    if (r0[b] < 0) return;
+    ok = hipEventSynchronize(p.done[b]) == hipSuccess && ok;
+    if (!j.up && ok) memcpy(j.host + (size_t)r0[b] * j.w, p.buf[b], (size_t)rows[b] * j.w * sizeof(double));
+    r0[b] = -1;
+  };
+  while (ok && !j.err.load(std::memory_order_relaxed)) {
+    const int q = j.next.fetch_add(1, std::memory_order_relaxed);
+    if (q >= j.runs) break;
+    finish(k);
+    if (!ok) break;
+    r0[k] = q * j.run;
+    rows[k] = total - r0[k] < j.run ? total - r0[k] : j.run;
+    if (j.up) memcpy(p.buf[k], j.host + (size_t)r0[k] * j.w, (size_t)rows[k] * j.w * sizeof(double));
+    ok = io_launch(j, p.buf[k], r0[k], rows[k]) && hipEventRecord(p.done[k], j.c->stream) == hipSuccess;
+    if (!ok) r0[k] = -1;
+    k ^= 1;
+  }
+  finish(k);
+  finish(k ^ 1);
+  if (!ok) j.err.store(1, std::memory_order_relaxed);
+}
+
+// row by row with strided copies: device pointers given in place of host
+// arrays, and where no pinned memory is to be had
+static int copy_planes_strided(cueva_ctx* c, double* const* planes, int n, double* host, bool up) {
   const Geom& g = c->g;
-  const size_t hw = (size_t)(g.imax + 13), hh = (size_t)(g.jmax + 13);
+  const size_t hw = (size_t)(g.imax + 13), hh = (size_t)(g.jmax + 13), row = hw * sizeof(double);
   for (int k = 0; k < n; k++) {
-    HIPCHK(hipMemcpy2DAsync(dst[k] + 2, (size_t)g.pitch * sizeof(double), host + (size_t)k * hw * hh,
-                            hw * sizeof(double), hw * sizeof(double), hh, hipMemcpyHostToDevice, c->stream));
+    double* h = host + (size_t)k * hw * hh;
+    const size_t pitch = (size_t)g.pitch * sizeof(double);
+    if (up)
+      HIPCHK(hipMemcpy2DAsync(planes[k] + 2, pitch, h, row, row, hh, hipMemcpyHostToDevice, c->stream));
+    else
+      HIPCHK(hipMemcpy2DAsync(h, row, planes[k] + 2, pitch, row, hh, hipMemcpyDeviceToHost, c->stream));
   }
   return CUEVA_OK;
 }
 
-static int copy_planes_d2h(cueva_ctx* c, double* const* src, int n, double* host) {
-  const Geom& g = c->g;
-  const size_t hw = (size_t)(g.imax + 13), hh = (size_t)(g.jmax + 13);
-  for (int k = 0; k < n; k++) {
-    HIPCHK(hipMemcpy2DAsync(host + (size_t)k * hw * hh, hw * sizeof(double), src[k] + 2,
-                            (size_t)g.pitch * sizeof(double), hw * sizeof(double), hh, hipMemcpyDeviceToHost,
-                            c->stream));
+// n planes (at most 32) up from or down to a host array; the caller's array is
+// read or written in full when this returns
+static int copy_planes(cueva_ctx* c, double* const* planes, int n, double* host, bool up) {
+  hipPointerAttribute_t at;
+  const hipError_t ae = hipPointerGetAttributes(&at, host);
+  if (ae != hipSuccess) (void)hipGetLastError();
+  if (ae == hipSuccess && at.type == hipMemoryTypeDevice) return copy_planes_strided(c, planes, n, host, up);
+  IoJob j;
+  j.c = c;
+  memset(&j.pl, 0, sizeof(j.pl));
+  j.pl.n = n;
+  for (int k = 0; k < n; k++) j.pl.a[k] = planes[k];
+  j.host = host;
+  j.up = up;
+  j.w = c->g.imax + 13;
+  j.hh = c->g.jmax + 13;
+  const int total = n * j.hh;
+  const size_t row = (size_t)j.w * sizeof(double), bytes = row * (size_t)total;
+  // two runs for a small transfer (one copied while the other is placed)
+  size_t run = (total + 1) / 2;
+  if (run * row > IO_CHUNK) run = IO_CHUNK / row;
+  j.run = (int)run;
+  j.runs = (int)((total + run - 1) / run);
+  j.next = 0;
+  j.err = 0;
+  if (hipGetDevice(&j.dev) != hipSuccess) return CUEVA_E_HIP;
+  int threads = 1;
+  if (bytes > 4 * IO_CHUNK) {
+    cpu_set_t set;
+    const int cpus = sched_getaffinity(0, sizeof(set), &set) == 0 ? CPU_COUNT(&set) : 1;
+    threads = std::max(1, std::min({IO_MAX_THREADS, cpus / 2, j.runs / 2}));
   }
-  return CUEVA_OK;
+  for (int t = 0; t < threads; t++)
+    if (!io_reserve(c->io[t], run * row)) {
+      if (t == 0) return copy_planes_strided(c, planes, n, host, up);
+      threads = t;
+      break;
+    }
+  std::thread th[IO_MAX_THREADS];
+  for (int t = 1; t < threads; t++) {
+    try {
+      th[t] = std::thread([&j, c, t]() {
+        if (hipSetDevice(j.dev) == hipSuccess) io_work(j, c->io[t]);
+      });
+    } catch (const std::exception&) {  // no more threads: the others take its runs
+      break;
+    }
+  }
+  io_work(j, c->io[0]);
+  for (int t = 1; t < threads; t++)
+    if (th[t].joinable()) th[t].join();
+  return j.err ? CUEVA_E_HIP : CUEVA_OK;
+}
+
+static int copy_planes_h2d(cueva_ctx* c, double* const* dst, int n, const double* host) {
+  return copy_planes(c, dst, n, const_cast<double*>(host), true);
+}
+
+static int copy_planes_d2h(cueva_ctx* c, double* const* src, int n, double* host) {
+  return copy_planes(c, src, n, host, false);
 }
 
 static dim3 interior_grid(const Geom& g, dim3 blk) {

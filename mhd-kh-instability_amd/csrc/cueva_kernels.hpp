@@ -63,6 +63,41 @@ __global__ void __launch_bounds__(256) k_fill_ghosts(Geom g, PlaneList pl, Statu
 // at most 12 (65536 + 13) + 12 (65536 + 1): fits 32 bits
 inline int64_t ghost_count(const Geom& g) { return 12LL * (g.imax + 13) + 12LL * (g.jmax + 1); }
 
+// Rows r0 .. r0+rows-1 of a host-layout array (n planes of hh rows of w
+// doubles, one after the other) between a buffer that holds just them and the
+// device planes.  Block 64 x 4: a wavefront moves 256 columns of one row, four
+// loads in flight a lane, since the buffer is host memory across the link.
+__global__ void __launch_bounds__(256) k_rows_to_planes(const double* __restrict__ buf, PlaneList pl, int w, int hh,
+                                                        int pitch, int r0, int rows) {
+  const int r = (int)(blockIdx.y * 4 + threadIdx.y);
+  if (r >= rows) return;
+  const int p = (r0 + r) / hh, j = (r0 + r) - p * hh, x = (int)(blockIdx.x * 256 + threadIdx.x);
+  const double* s = buf + (int64_t)r * w;
+  double* d = pl.a[p] + (int64_t)j * pitch + 2;
+  double v[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    if (x + 64 * k < w) v[k] = s[x + 64 * k];
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    if (x + 64 * k < w) d[x + 64 * k] = v[k];
+}
+__global__ void __launch_bounds__(256) k_planes_to_rows(double* __restrict__ buf, PlaneList pl, int w, int hh,
+                                                        int pitch, int r0, int rows) {
+  const int r = (int)(blockIdx.y * 4 + threadIdx.y);
+  if (r >= rows) return;
+  const int p = (r0 + r) / hh, j = (r0 + r) - p * hh, x = (int)(blockIdx.x * 256 + threadIdx.x);
+  const double* s = pl.a[p] + (int64_t)j * pitch + 2;
+  double* d = buf + (int64_t)r * w;
+  double v[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    if (x + 64 * k < w) v[k] = s[x + 64 * k];
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    if (x + 64 * k < w) d[x + 64 * k] = v[k];
+}
+
 // ---------------------------------------------------------------------------
 // pointwise kernels over the interior [0,imax] x [0,jmax]
 // ---------------------------------------------------------------------------
