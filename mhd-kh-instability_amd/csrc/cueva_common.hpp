@@ -94,6 +94,7 @@ struct Scheme {
   // with the MIRK coefficients cm_1, cm_2, cm_4 (:233-235)
   int mirk;
   int rec_prim;  // stage primitive recovery (parameters.f95:23)
+  int stream;    // outputs stored past the caches: 1 the marching kernel's, 2 the recovery pass's too
   double cm1, cm2, cm4;
 };
 

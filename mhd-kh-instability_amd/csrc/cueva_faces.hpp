@@ -771,20 +771,18 @@ k_faces_march(MarchArgs args) {
       const int64_t k = g.at(i, j);
       const Rhs r = rhs_of<T, false>(P, S, k, dfx, dfy);  // never with REC_PRIM = 1
       if constexpr (!FINAL) {
-#pragma unroll
-        for (int t = 0; t < R_N; t++) P.rhs[l][t][k] = r.r[t];
+        put_planes<R_N>(P.rhs[l], k, r.r, S.stream > 0);
         // the next stage's state of this point (pointwise in U^n and the
         // stage right-hand sides, the last of which is still in registers)
         double sv[S_N];
         stage_point(P, S, l + 1, k, false, P.p[P_VX][k], P.p[P_VY][k], P.p[P_VZ][k], P.p[P_EX][k], P.p[P_EY][k],
                     P.p[P_EZ][k], P.p[P_BX][k], P.p[P_BY][k], P.p[P_BZ][k], P.p[P_RHO][k], P.p[P_P][k],
                     P.p[P_PSI][k], P.p[P_PHI][k], P.p[P_Q][k], sv, &r);
-        store_stage(P.sn, k, sv);
+        store_stage(P.sn, k, sv, S.stream > 0);
       } else {
         double nu[A_N];
         final_update_from(P, S, k, r, nu);
-#pragma unroll
-        for (int a = 0; a < A_N; a++) P.rhs[l][a][k] = nu[a];
+        put_planes<A_N>(P.rhs[l], k, nu, S.stream > 0);
         if constexpr (C2P) recover_point(P, S, st, i, j, k, nu, A.stage0);
       }
     }

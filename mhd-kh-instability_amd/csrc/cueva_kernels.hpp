@@ -483,7 +483,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))
   if (fallback) atomicAdd(&sr.st->fallback, 1ULL);
   if (code) { report(sr, code, i, j, 1); return; }
   c2p_count(sr, i, j, out);
-  c2p_store_out(P, k, out);
+  c2p_store_out(P, S, k, out);
 }
 
 }  // namespace cueva

@@ -247,11 +247,10 @@ __global__ void __launch_bounds__(256) k_c2p_learned(Geom g, Planes P, Scheme S,
   using namespace mlp;
   if (halted(sr)) return;
   const int lane = threadIdx.x & 63;
-  const int ni = g.imax + 1;
-  const int64_t ncell = (int64_t)ni * (g.jmax + 1);
-  const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool valid = n < ncell;
-  const int j = valid ? (int)(n / ni) : 0, i = valid ? (int)(n - (int64_t)j * ni) : 0;
+  const int i0 = (int)(blockIdx.x * 64 + threadIdx.x), j0 = (int)(blockIdx.y * 4 + threadIdx.y);
+  const bool valid = i0 <= g.imax && j0 <= g.jmax;
+  // the network runs wavefront-wide: points past the edge compute on an edge point
+  const int i = i0 <= g.imax ? i0 : g.imax, j = j0 <= g.jmax ? j0 : g.jmax;
   const int64_t k = g.at(i, j);
   C2PIn in;
   in.d = P.c[C_D][k]; in.tau = P.c[C_TAU][k];
@@ -268,18 +267,18 @@ __global__ void __launch_bounds__(256) k_c2p_learned(Geom g, Planes P, Scheme S,
   if (fallback) atomicAdd(&sr.st->fallback, 1ULL);
   if (code) { report(sr, code, i, j, 1); return; }
   c2p_count(sr, i, j, out);
-  c2p_store_out(P, k, out);
+  c2p_store_out(P, S, k, out);
   if (STAGE0) stage0_after_c2p(P, S, k, in, out);
 }
 
 hipError_t launch_c2p_learned(hipStream_t s, const Geom& g, const Planes& P, const Scheme& S, const float* wp,
                               const StatusRef& sr, bool stage0) {
-  const int64_t ncell = (int64_t)(g.imax + 1) * (g.jmax + 1);
-  const dim3 grid((unsigned)((ncell + 255) / 256));
+  // rows of 64 points, each starting at a multiple of 64 columns: whole cache lines
+  const dim3 grid((unsigned)((g.imax + 64) / 64), (unsigned)((g.jmax + 4) / 4)), blk(64, 4);
   if (stage0)
-    hipLaunchKernelGGL(k_c2p_learned<true>, grid, dim3(256), 0, s, g, P, S, wp, sr);
+    hipLaunchKernelGGL(k_c2p_learned<true>, grid, blk, 0, s, g, P, S, wp, sr);
   else
-    hipLaunchKernelGGL(k_c2p_learned<false>, grid, dim3(256), 0, s, g, P, S, wp, sr);
+    hipLaunchKernelGGL(k_c2p_learned<false>, grid, blk, 0, s, g, P, S, wp, sr);
   return hipGetLastError();
 }
 

@@ -10,6 +10,29 @@ namespace cueva {
 
 struct Rhs { double r[R_N]; };
 
+// Values that no later part of the launch reads, n planes at offset k.  On
+// large grids they are stored past the caches (non-temporal, Scheme::stream):
+// the marching kernel's 34 output planes a cell otherwise push out the stencil
+// rows that its next tile step reads again.  With against without, at
+// 2048x4096: fabric traffic of an FP32 stage launch 7.3 against 7.9 GB, step
+// FP64 HLLC 5.07 against 5.13 ms, mixed HLL 3.98 against 4.09; mixed HLLE + MP7
+// at 1024x2048 1.20 against 1.24.  Small grids, whose planes the 256 MB
+// Infinity Cache keeps from launch to launch, lose by it (HLL + MC at 300x700
+// 201 against 186 us).
+template <int N> __device__ inline void put_planes(double* const* p, int64_t k, const double* v, bool stream) {
+  if (stream) {
+    // the empty statements keep the compiler from merging the two branches'
+    // stores into one that is not streamed
+    asm volatile("");
+#pragma unroll
+    for (int t = 0; t < N; t++) __builtin_nontemporal_store(v[t], &p[t][k]);
+    asm volatile("");
+  } else {
+#pragma unroll
+    for (int t = 0; t < N; t++) p[t][k] = v[t];
+  }
+}
+
 template <typename FT> __device__ inline FT ddx(const Scheme& S, FT a) {
   return S.div_exact ? a * (FT)S.inv_dx : a / (FT)S.dx;
 }
@@ -216,10 +239,10 @@ __device__ inline void stage_point(const Planes& P, const Scheme& S, int l, int6
   out[S_JX] = jx; out[S_JY] = jy; out[S_JZ] = jz;
 }
 
-__device__ inline void store_stage(double* const* s, int64_t k, const double* v) {
-#pragma unroll
-  for (int t = 0; t < S_N; t++)
-    if (t < S_EXA || t > S_EZA) s[t][k] = v[t];
+__device__ inline void store_stage(double* const* s, int64_t k, const double* v, bool stream = false) {
+  static_assert(S_EXA == 5 && S_EZA == 7, "the unused E* planes are 5 to 7");
+  put_planes<S_EXA>(s, k, v, stream);
+  put_planes<S_N - S_EZA - 1>(s + S_EZA + 1, k, v + S_EZA + 1, stream);
 }
 
 // primitive recovery of one point (Cardano, 12_varprimitive.f95) and the
@@ -231,10 +254,10 @@ __device__ inline void c2p_count(const StatusRef& sr, int i, int j, const C2POut
 }
 
 // the recovered primitives of one point and its W (12_varprimitive.f95:793-802)
-__device__ inline void c2p_store_out(const Planes& P, int64_t k, const C2POut& o) {
+__device__ inline void c2p_store_out(const Planes& P, const Scheme& S, int64_t k, const C2POut& o) {
 #pragma clang fp contract(off)
-  P.pn[0][k] = o.vx; P.pn[1][k] = o.vy; P.pn[2][k] = o.vz;
-  P.pn[3][k] = o.rho; P.pn[4][k] = o.p;
+  const double v[5] = {o.vx, o.vy, o.vz, o.rho, o.p};
+  put_planes<5>(P.pn, k, v, S.stream > 1);
   P.c[C_W][k] = 1.0 / sqrt(1.0 - ((sq(o.vx) + sq(o.vy)) + sq(o.vz)));
 }
 
@@ -243,7 +266,7 @@ __device__ inline bool c2p_apply(const Planes& P, const Scheme& S, const StatusR
   int code = c2p_cardano_full(S.gamma, S.eps1, in, o, S.crmath != 0);
   if (code) { report(sr, code, i, j, 1); return false; }
   c2p_count(sr, i, j, o);
-  c2p_store_out(P, k, o);
+  c2p_store_out(P, S, k, o);
   return true;
 }
 
@@ -278,7 +301,7 @@ __device__ inline void recover_point(const Planes& P, const Scheme& S, const Sta
     double sv[S_N];
     stage_point(P, S, 0, k, false, o.vx, o.vy, o.vz, in.ex, in.ey, in.ez, in.bx, in.by, in.bz, o.rho, o.p,
                 nu[A_PSI], nu[A_PHI], nu[A_Q], sv);
-    store_stage(P.sn, k, sv);
+    store_stage(P.sn, k, sv, S.stream > 0);
   }
 }
 
@@ -288,7 +311,7 @@ __device__ inline void stage0_after_c2p(Planes& P, const Scheme& S, int64_t k, c
   double out[S_N];
   stage_point(P, S, 0, k, false, o.vx, o.vy, o.vz, in.ex, in.ey, in.ez, in.bx, in.by, in.bz, o.rho, o.p,
               P.p[P_PSI][k], P.p[P_PHI][k], P.p[P_Q][k], out);
-  store_stage(P.s, k, out);
+  store_stage(P.s, k, out, S.stream > 1);
 }
 
 }  // namespace cueva
