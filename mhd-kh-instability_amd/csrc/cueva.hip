@@ -373,6 +373,28 @@ extern "C" int cueva_create(const cueva_params* p, cueva_ctx** out) {
       c->P.pint[l] = take();
       c->P.hint[l] = take();
     }
+  S.full = 1;
+  // the mixed marching step's FP32 copies of the stencil planes: two to a
+  // face-flux plane, which that step does not use (fx[0..4] take part in the
+  // recovery's exchange, take_recovered)
+  if (p->precision == CUEVA_MIXED && c->march && !p->rec_prim) {
+    int h = 0;
+    auto half = [&]() {
+      const int t = h++;
+      double* q = t / 2 < FX_N - 5 ? c->P.fx[5 + t / 2] : c->P.fy[t / 2 - (FX_N - 5)];
+      return (float*)q + (t & 1 ? g.plane : 0);
+    };
+    for (int k = 0; k < S_JZ; k++)
+      if (k < S_EXA || k > S_EZA) {
+        c->P.sf[k] = half();
+        c->P.snf[k] = half();
+      }
+    for (int k = 0; k < K_N; k++) {
+      c->P.kf[k] = half();
+      c->P.knf[k] = half();
+    }
+    static_assert(2 * (S_JZ - 3 + K_N) <= 2 * (FX_N - 5 + FY_N), "the FP32 copies fit the face-flux planes");
+  }
   recover_in_place(c->P);
   // every plane pointer the kernels receive must lie inside the allocation
   {
@@ -637,23 +659,22 @@ static StatusRef sref(cueva_ctx* c, int l, bool record = false, bool fused = fal
   return r;
 }
 
-// copy every ghost point of the planes from its interior source point; the
-// last nzero planes (at most 32) are set to 0 there instead
+// copy every ghost point of the planes from its interior source point
+static int fill_ghosts(cueva_ctx* c, const PlaneList& pl) {
+  const int64_t cnt = ghost_count(c->g);
+  LAUNCH(K_GHOSTS, k_fill_ghosts, dim3((unsigned)((cnt + 255) / 256), ghost_groups(pl)), dim3(256), c->g, pl, sref(c, 0));
+  return launch_ok() ? CUEVA_E_HIP : CUEVA_OK;
+}
+
+// the same for n FP64 planes, at most 32 of them; the last nzero are set to 0 there instead
 static int fill_ghosts(cueva_ctx* c, double* const* planes, int n, int nzero = 0) {
-  const StatusRef sr = sref(c, 0);
   PlaneList pl;
   memset(&pl, 0, sizeof(pl));
-  for (int start = 0; start < n; start += 32) {
-    pl.n = n - start < 32 ? n - start : 32;
-    pl.nzero = start + pl.n == n ? nzero : 0;
-    for (int k = 0; k < pl.n; k++) pl.a[k] = planes[start + k];
-    int64_t cnt = ghost_count(c->g);
-    LAUNCH(K_GHOSTS, k_fill_ghosts,
-           dim3((unsigned)((cnt + 255) / 256), (unsigned)((pl.n + GHOST_PLANES - 1) / GHOST_PLANES)), dim3(256), c->g, pl,
-           sr);
-    if (launch_ok()) return CUEVA_E_HIP;
-  }
-  return CUEVA_OK;
+  if (n > (int)(sizeof(pl.a) / sizeof(pl.a[0]))) return CUEVA_E_ARG;
+  pl.n = n;
+  pl.nzero = nzero;
+  for (int k = 0; k < n; k++) pl.a[k] = planes[k];
+  return fill_ghosts(c, pl);
 }
 
 extern "C" int cueva_upload_prims(cueva_ctx* c, const double* prims14) {
@@ -911,6 +932,33 @@ extern "C" int cueva_electricfield(cueva_ctx* c) {
   return launch_ok();
 }
 
+// ghost band of a stage state formed at the interior points only: a copy of
+// the source point's (the state is pointwise in the point's own data), except
+// J under HLLE and HLL+MCL, which the reference keeps 0 there
+// (24_boundary_flux_conserved.f95:13).  Adds its planes to pl: the mixed form's
+// stencils read FP32 copies, and its FP64 planes take part only with `full`
+// (the state that stays after the call).
+static void stage_ghost_list(const cueva_ctx* c, bool full, PlaneList& pl) {
+  static const int st[17] = {S_PSI, S_PHI, S_BX, S_BY, S_BZ, S_Q, S_D, S_TAU, S_SX, S_SY, S_SZ,
+                             S_EX, S_EY, S_EZ, S_JX, S_JY, S_JZ};
+  const bool zero_j = !j_ghosts_filled(c->prm.flux_solver);
+  if (!c->P.sf[0] || full) {
+    const int np = full ? 17 : 16;  // J_z is read by nothing
+    for (int k = 0; k < np; k++) pl.a[pl.n++] = c->P.s[st[k]];
+    pl.nzero = zero_j ? np - 14 : 0;
+  }
+  if (c->P.sf[0]) {
+    for (int k = 0; k < 16; k++) pl.f[pl.nf++] = c->P.sf[st[k]];
+    pl.nfzero = zero_j ? 2 : 0;
+  }
+}
+
+static int stage_halo(const cueva_ctx* c) { return (c->rec_order - 1) / 2 + 1; }  // stencil radius K plus the face offset
+static dim3 stage_grid(const Geom& g, int halo) {
+  return dim3((unsigned)((g.imax + 1 + 2 * halo + BLK.x - 1) / BLK.x),
+              (unsigned)((g.jmax + 1 + 2 * halo + BLK.y - 1) / BLK.y));
+}
+
 // Wait for the device and read the status words.  A first failure found here
 // becomes the context's (code and where: step, stage, i, j); if it arose in
 // the fused step, the plane roles go back to those the failing launch ran
@@ -932,6 +980,23 @@ static int read_status(cueva_ctx* c, DevStatus* h) {
         if (lr.fused) {
           c->P = lr.P;
           recover_in_place(c->P);
+          // the failing launch's stage state in full (the marching step keeps
+          // what its launches read): formed again from the step's start,
+          // which the later launches left alone
+          if (c->march && lr.l >= 1) {
+            const int halo = stage_halo(c);
+            StatusRef none = {};
+            none.st = c->dst;  // number 0: no earlier launch halts it
+            hipLaunchKernelGGL(k_stage_fused, stage_grid(c->g, halo), BLK, 0, c->stream, c->g, c->P, c->S, lr.l - 1, halo,
+                               none);
+            PlaneList pl;
+            memset(&pl, 0, sizeof(pl));
+            stage_ghost_list(c, true, pl);
+            hipLaunchKernelGGL(k_fill_ghosts, dim3((unsigned)((ghost_count(c->g) + 255) / 256), ghost_groups(pl)), dim3(256),
+                               0, c->stream, c->g, pl, none);
+            HIPCHK(hipGetLastError());
+            HIPCHK(hipStreamSynchronize(c->stream));
+          }
         }
         break;
       }
@@ -944,19 +1009,21 @@ static int read_status(cueva_ctx* c, DevStatus* h) {
 // cueva_step; stage0: also the next step's stage-0 state at the interior.
 // snap: the plane roles a failure restores (default: those of this launch)
 static int launch_c2p(cueva_ctx* c, bool fused, int cls = K_OTHER, bool stage0 = false,
-                      const Planes* snap = nullptr) {
+                      const Planes* snap = nullptr, int full = 1) {
+  Scheme S = c->S;
+  S.full = full;
   const StatusRef sr = sref(c, c->S.lmax, true, fused, snap);
   if (c->prm.c2p_mode == CUEVA_C2P_LEARNED) {
     if (!c->has_mlp) return CUEVA_E_ARG;
     prof_begin(c, cls);
-    hipError_t e = launch_c2p_learned(c->stream, c->g, c->P, c->S, c->mlpw, sr, stage0);
+    hipError_t e = launch_c2p_learned(c->stream, c->g, c->P, S, c->mlpw, sr, stage0);
     prof_end(c);
     return e == hipSuccess ? CUEVA_OK : CUEVA_E_HIP;
   }
   if (stage0)
-    LAUNCH(cls, k_c2p<true>, interior_grid(c->g, BLK), BLK, c->g, c->P, c->S, sr);
+    LAUNCH(cls, k_c2p<true>, interior_grid(c->g, BLK), BLK, c->g, c->P, S, sr);
   else
-    LAUNCH(cls, k_c2p<false>, interior_grid(c->g, BLK), BLK, c->g, c->P, c->S, sr);
+    LAUNCH(cls, k_c2p<false>, interior_grid(c->g, BLK), BLK, c->g, c->P, S, sr);
   return launch_ok() ? CUEVA_E_HIP : CUEVA_OK;
 }
 
@@ -994,20 +1061,31 @@ static int march_waves(const cueva_ctx* c) {
   return march_block_waves(c->prm.precision == CUEVA_MIXED, c->prm.flux_solver);
 }
 
-// ghost band of a stage state formed at the interior points only: a copy of
-// the source point's (the state is pointwise in the point's own data), except
-// J under HLLE and HLL+MCL, which the reference keeps 0 there
-// (24_boundary_flux_conserved.f95:13);
 // with_prims: the primitive planes' ghosts in the same launch
-static int fill_stage_ghosts(cueva_ctx* c, bool with_prims = false) {
-  double* list[P_N + 17];
-  int n = 0;
-  if (with_prims)
-    for (int k = 0; k < P_N; k++) list[n++] = c->P.p[k];
-  const int st[17] = {S_PSI, S_PHI, S_BX, S_BY, S_BZ, S_Q, S_D, S_TAU, S_SX, S_SY, S_SZ,
-                      S_EX, S_EY, S_EZ, S_JX, S_JY, S_JZ};
-  for (int k = 0; k < 17; k++) list[n++] = c->P.s[st[k]];
-  return fill_ghosts(c, list, n, j_ghosts_filled(c->prm.flux_solver) ? 0 : 3);
+static int fill_stage_ghosts(cueva_ctx* c, bool full, bool with_prims = false) {
+  PlaneList pl;
+  memset(&pl, 0, sizeof(pl));
+  if (with_prims) {
+    for (int k = 0; k < P_N; k++) pl.a[pl.n++] = c->P.p[k];
+    if (c->P.kf[0])
+      for (int k = 0; k < K_N; k++) pl.f[pl.nf++] = c->P.kf[k];
+  }
+  stage_ghost_list(c, full, pl);
+  return fill_ghosts(c, pl);
+}
+
+// the stage state just formed takes the place of the one read
+static void swap_stage(cueva_ctx* c) {
+  for (int t = 0; t < S_N; t++) {
+    std::swap(c->P.s[t], c->P.sn[t]);
+    std::swap(c->P.sf[t], c->P.snf[t]);
+  }
+}
+
+// Whether the state of stage l of step h out of nsteps (0-based) stays after
+// the call: it is then kept in full (store_stage).
+static int stays(const cueva_ctx* c, int l, int h, int nsteps) {
+  return !c->march || (l == c->S.lmax - 1 && h == nsteps - 1);
 }
 
 // U^{n+1}, left by the last marching launch in rhs[L][0..13], becomes the
@@ -1044,6 +1122,7 @@ static void take_recovered(cueva_ctx* c) {
     c->P.fx[q] = t;
     c->P.fxf[q] = (float*)t;
   }
+  for (int q = 0; q < K_N; q++) std::swap(c->P.kf[q], c->P.knf[q]);
   recover_in_place(c->P);
 }
 
@@ -1101,9 +1180,10 @@ static int march_seg(cueva_ctx* c, bool fin, bool c2p) {
   return seg;
 }
 
+// full: the stage state it forms is kept in FP64 in full (mixed form)
 // c2p (last stage only): with the primitive recovery (to P.pn) and, with
 // stage0, the next step's stage-0 state (to P.sn)
-static int launch_march(cueva_ctx* c, int l, bool fin, bool c2p = false, bool stage0 = false) {
+static int launch_march(cueva_ctx* c, int l, bool fin, int full, bool c2p = false, bool stage0 = false) {
   // its face solves and right-hand side read the t^n primitives (no stage
   // kinematics: REC_PRIM = 1 runs the per-subroutine sequence)
   if (c->prm.rec_prim) return CUEVA_E_ARG;
@@ -1120,6 +1200,7 @@ static int launch_march(cueva_ctx* c, int l, bool fin, bool c2p = false, bool st
   ma.P = c->P;
   ma.g = c->g;
   ma.S = c->S;
+  ma.S.full = full;
   ma.l = l;
   ma.seg = seg;
   ma.st = sref(c, l + 1, true, true);
@@ -1137,7 +1218,7 @@ static int routine_steps(cueva_ctx* c, int nsteps);
 
 extern "C" int cueva_step(cueva_ctx* c, int nsteps) {
   if (!c || nsteps < 0) return CUEVA_E_ARG;
-  const int halo = (c->rec_order - 1) / 2 + 1;  // stencil radius K plus the face offset
+  const int halo = stage_halo(c);
   const bool learned = c->prm.c2p_mode == CUEVA_C2P_LEARNED;
   if (learned && !c->has_mlp) return CUEVA_E_ARG;
   if (c->err) return c->err;
@@ -1165,9 +1246,10 @@ static int fused_steps(cueva_ctx* c, int nsteps, int halo, bool learned) {
       // the marching path forms stage l >= 1 in the previous stage's face pass
       const bool have_stage = c->march && (l > 0 || s0_ready);
       if (!have_stage) {
-        dim3 gs((unsigned)((g.imax + 1 + 2 * halo + BLK.x - 1) / BLK.x),
-                (unsigned)((g.jmax + 1 + 2 * halo + BLK.y - 1) / BLK.y));
-        LAUNCH(K_STAGE, k_stage_fused, gs, BLK, c->g, c->P, c->S, l, halo, sref(c, l + 1));
+        const dim3 gs = stage_grid(g, halo);
+        Scheme S = c->S;
+        S.full = stays(c, l, h, nsteps);
+        LAUNCH(K_STAGE, k_stage_fused, gs, BLK, c->g, c->P, S, l, halo, sref(c, l + 1));
         if (launch_ok()) return CUEVA_E_HIP;
       }
       if (c->march) {
@@ -1177,15 +1259,13 @@ static int fused_steps(cueva_ctx* c, int nsteps, int halo, bool learned) {
         const bool in_kernel = last && !learned && c->c2p_in_march;
         const Planes pre = c->P;
         if (last) recover_to_scratch(c);
-        int rc = launch_march(c, l, last, in_kernel, in_kernel && h + 1 < nsteps && !c->prm.primitive_rec);
+        // the state that this launch forms: the next stage's, or the next step's first
+        const int full = last ? stays(c, 0, h + 1, nsteps) : stays(c, l + 1, h, nsteps);
+        int rc = launch_march(c, l, last, full, in_kernel, in_kernel && h + 1 < nsteps && !c->prm.primitive_rec);
         if (rc) return rc;
         if (!last) {
-          for (int t = 0; t < S_N; t++) {
-            double* x = c->P.s[t];
-            c->P.s[t] = c->P.sn[t];
-            c->P.sn[t] = x;
-          }
-          if ((rc = fill_stage_ghosts(c))) return rc;
+          swap_stage(c);
+          if ((rc = fill_stage_ghosts(c, full))) return rc;
           continue;
         }
         adopt_update(c, l);
@@ -1193,17 +1273,13 @@ static int fused_steps(cueva_ctx* c, int nsteps, int halo, bool learned) {
         // (not when the next step first re-forms the primitives)
         const bool fuse = h + 1 < nsteps && !c->prm.primitive_rec;
         if (!in_kernel) {
-          if ((rc = launch_c2p(c, true, K_FINAL, fuse, &pre))) return rc;
+          if ((rc = launch_c2p(c, true, K_FINAL, fuse, &pre, full))) return rc;
         } else if (fuse) {
-          for (int t = 0; t < S_N; t++) {
-            double* x = c->P.s[t];
-            c->P.s[t] = c->P.sn[t];
-            c->P.sn[t] = x;
-          }
+          swap_stage(c);
         }
         take_recovered(c);
         // ghosts of the new primitives (and of the next stage-1 state)
-        if ((rc = fuse ? fill_stage_ghosts(c, true) : fill_ghosts(c, c->P.p, P_N))) return rc;
+        if ((rc = fuse ? fill_stage_ghosts(c, full, true) : fill_ghosts(c, c->P.p, P_N))) return rc;
         s0_ready = fuse;
         continue;
       }

@@ -30,6 +30,19 @@ struct Planes {
   double* c[C_N];
   double* s[S_N];
   double* sn[S_N];  // the next stage's state, written by the marching kernel while s is read
+  // mixed form, marching step: FP32 copies of what the stencils read (the
+  // stage state without J_z and the unused E*; the primitives' velocity,
+  // pressure and density in K_* order), and the set being written next; null
+  // otherwise.  The FP32 stencils convert every value they load, so the copies
+  // give the same bits for half the bytes: those launches ran at the fabric's
+  // copy rate (4.2-4.8 TB/s, 9 stencil rows of 21 FP64 planes for every 4 face
+  // rows).  2048x4096, copies against FP64 planes: face launches 2.71 against
+  // 3.42 ms a step, recovery pass 0.60 against 0.56 (more, narrower stores),
+  // step 3.37 against 4.04 ms; HLLE + MP7 at 1024x2048 0.94 against 1.20 ms.
+  float* sf[S_N];
+  float* snf[S_N];
+  float* kf[5];
+  float* knf[5];
   double* fx[FX_N];
   double* fy[FY_N];
   float* fxf[FX_N];  // the same memory as fx/fy, as FP32 planes (mixed form)
@@ -68,6 +81,17 @@ __device__ inline const double* kin_plane(const Planes& P, int q) {
   return P.kin[q] ? P.kin[q] : P.p[pq];
 }
 
+// the plane the stencils read for stage quantity k / kinematic quantity q, in
+// the storage type ST: the FP64 planes, or their FP32 copies
+template <typename ST> __device__ inline const ST* stage_src(const Planes& P, int k) {
+  if constexpr (sizeof(ST) == 4) return P.sf[k];
+  else return P.s[k];
+}
+template <typename ST, bool STAGE = true> __device__ inline const ST* kin_src(const Planes& P, int q) {
+  if constexpr (sizeof(ST) == 4) return P.kf[q];
+  else return kin_plane<STAGE>(P, q);
+}
+
 // the recovery writes in place
 inline void recover_in_place(Planes& P) {
   P.pn[0] = P.p[P_VX];
@@ -94,6 +118,7 @@ struct Scheme {
   // with the MIRK coefficients cm_1, cm_2, cm_4 (:233-235)
   int mirk;
   int rec_prim;  // stage primitive recovery (parameters.f95:23)
+  int full;      // the stage state is kept in full (store_stage): not inside the marching step
   int stream;    // outputs stored past the caches: 1 the marching kernel's, 2 the recovery pass's too
   double cm1, cm2, cm4;
 };

@@ -32,11 +32,12 @@
 
 namespace cueva {
 
-// Stencils loaded ahead of the one being reconstructed.  FP64 (2 waves per
-// SIMD, HLLC + MP5 at 2048x4096, step with 0 / 1 / 2 / 3): 6.6 / 5.53 / 5.19 /
-// 5.12 ms.  FP32 takes two at 3 waves per SIMD (4.16 ms; one at 3 waves 4.25,
-// one at 4 waves, which spill, 4.46, three at 2 waves 4.15).
-template <typename T> constexpr int face_ahead() { return sizeof(T) == 8 ? 3 : 2; }
+// Stencils loaded ahead of the one being reconstructed, by the type of the
+// planes they are loaded from.  FP64 planes (FP64 form, 2 waves per SIMD, HLLC
+// + MP5 at 2048x4096, step with 0 / 1 / 2 / 3): 6.6 / 5.53 / 5.19 / 5.12 ms.
+// FP32 planes (mixed form, 3 waves per SIMD, 2 / 3 / 4): 3.49 / 3.40 / 3.37
+// (5 at 2 waves 3.37; 4 waves per SIMD with 2 spill, 3.61).
+template <typename ST> constexpr int face_ahead() { return sizeof(ST) == 8 ? 3 : 4; }
 
 // launch grid of k_faces over the face pairs [-1,imax] x [-1,jmax]
 inline dim3 faces_grid(const Geom& g, dim3 blk) {
@@ -58,7 +59,7 @@ inline dim3 faces_grid(const Geom& g, dim3 blk) {
 // registers and each lane adds only its 32-bit byte offset within the row
 // (global loads take a scalar base, a 32-bit lane offset and a constant).
 struct Cell {
-  uint32_t vo;   // byte offset of column i in its row
+  uint32_t vo;   // byte offset of column i in its row of an FP64 plane
   int64_t ro;    // first element of row j (the same for every lane)
   int pitch;
 };
@@ -66,15 +67,15 @@ __device__ inline Cell cell_of(const Geom& g, int i, int j) {
   return {(uint32_t)(i + 8) * 8u, (int64_t)(__builtin_amdgcn_readfirstlane(j) + GH) * g.pitch, g.pitch};
 }
 // element (i + DI, j + dj)
-template <int DI = 0> __device__ inline double at_cell(const double* __restrict__ a, const Cell& c, int dj = 0) {
+template <int DI = 0, typename ST> __device__ inline ST at_cell(const ST* __restrict__ a, const Cell& c, int dj = 0) {
   const char* row = (const char*)(a + (c.ro + (int64_t)dj * c.pitch));
-  return *(const double*)(row + c.vo + DI * 8);
+  return *(const ST*)(row + (sizeof(ST) == 8 ? c.vo : c.vo >> 1) + DI * (int)sizeof(ST));
 }
 
-// the 2K+2 values of one quantity across the face, as loaded (FP64)
-template <int ORD> struct Sten { double v[2 * MPc<ORD>::K + 2]; };
-template <int ORD, int DIR, int... T>
-__device__ inline void sten_load(const double* __restrict__ a, const Cell& c, Sten<ORD>& s,
+// the 2K+2 values of one quantity across the face, as loaded
+template <int ORD, typename ST> struct Sten { ST v[2 * MPc<ORD>::K + 2]; };
+template <int ORD, int DIR, typename ST, int... T>
+__device__ inline void sten_load(const ST* __restrict__ a, const Cell& c, Sten<ORD, ST>& s,
                                  std::integer_sequence<int, T...>) {
   constexpr int K = MPc<ORD>::K;
   ((s.v[T] = DIR == 0 ? at_cell<DIR == 0 ? T - K : 0>(a, c) : at_cell(a, c, T - K)), ...);
@@ -84,15 +85,15 @@ __device__ inline void sten_load(const double* __restrict__ a, const Cell& c, St
 // kinematics first (the fallbacks couple the two faces of a pair)
 enum { F_VX, F_VY, F_VZ, F_P, F_RHO, F_PSI, F_PHI, F_EX, F_EY, F_EZ, F_BX, F_BY, F_BZ, F_Q, F_D, F_TAU, F_SX, F_SY,
        F_SZ, F_JN, F_NQ };
-template <int F, int DIR, bool STAGE_KIN> __device__ inline const double* face_plane(const Planes& P) {
+template <int F, int DIR, bool STAGE_KIN, typename ST> __device__ inline const ST* face_plane(const Planes& P) {
   if constexpr (F <= F_RHO) {
     constexpr int q = F == F_VX ? K_VX : F == F_VY ? K_VY : F == F_VZ ? K_VZ : F == F_P ? K_P : K_RHO;
-    return kin_plane<STAGE_KIN>(P, q);
+    return kin_src<ST, STAGE_KIN>(P, q);
   } else {
     constexpr int s[15] = {S_PSI, S_PHI, S_EX, S_EY, S_EZ, S_BX, S_BY, S_BZ, S_Q, S_D, S_TAU, S_SX, S_SY, S_SZ,
                            DIR == 0 ? S_JX : S_JY};
     constexpr int k = s[F - F_PSI];
-    return P.s[k];
+    return stage_src<ST>(P, k);
   }
 }
 template <int F, typename T> __device__ inline T& face_slot(Side<T>& o) {
@@ -103,13 +104,13 @@ template <int F, typename T> __device__ inline T& face_slot(Side<T>& o) {
   return o.*m[F];
 }
 
-template <int ORD, int F, int DIR, bool STAGE_KIN>
-__device__ inline void face_load(const Planes& P, const Cell& c, Sten<ORD>& s) {
-  sten_load<ORD, DIR>(face_plane<F, DIR, STAGE_KIN>(P), c, s,
+template <int ORD, int F, int DIR, bool STAGE_KIN, typename ST>
+__device__ inline void face_load(const Planes& P, const Cell& c, Sten<ORD, ST>& s) {
+  sten_load<ORD, DIR>(face_plane<F, DIR, STAGE_KIN, ST>(P), c, s,
                       std::make_integer_sequence<int, 2 * MPc<ORD>::K + 2>());
 }
-template <int ORD, int F, typename T>
-__device__ inline void face_take(const Sten<ORD>& s, Side<T>& L, Side<T>& R) {
+template <int ORD, int F, typename ST, typename T>
+__device__ inline void face_take(const Sten<ORD, ST>& s, Side<T>& L, Side<T>& R) {
   constexpr int N = 2 * MPc<ORD>::K + 2;
   T v[N];
 #pragma unroll
@@ -122,11 +123,11 @@ __device__ inline void face_take(const Sten<ORD>& s, Side<T>& L, Side<T>& R) {
 // quantities are loaded before the current one is reconstructed: the
 // limiter's wavefront-wide branch keeps the compiler from moving loads across
 // it, and without this every quantity waited for its own loads.
-template <int ORD, int F0, int DIR, bool STAGE_KIN, typename T, int... S>
+template <int ORD, int F0, int DIR, bool STAGE_KIN, typename ST, typename T, int... S>
 __device__ inline void face_fields_seq(const Planes& P, const Cell& c, Side<T>& L, Side<T>& R,
                                        std::integer_sequence<int, S...>) {
-  constexpr int N = sizeof...(S), AH = face_ahead<T>();
-  Sten<ORD> b[AH + 1];
+  constexpr int N = sizeof...(S), AH = face_ahead<ST>();
+  Sten<ORD, ST> b[AH + 1];
   auto pre = [&](auto t) {
     if constexpr (t() < AH && t() < N) face_load<ORD, F0 + t(), DIR, STAGE_KIN>(P, c, b[t()]);
   };
@@ -138,9 +139,9 @@ __device__ inline void face_fields_seq(const Planes& P, const Cell& c, Side<T>& 
   (pre(std::integral_constant<int, S>()), ...);
   (one(std::integral_constant<int, S>()), ...);
 }
-template <int ORD, int F0, int F1, int DIR, bool STAGE_KIN, typename T>
+template <int ORD, int F0, int F1, int DIR, bool STAGE_KIN, typename ST, typename T>
 __device__ inline void face_fields(const Planes& P, const Cell& c, Side<T>& L, Side<T>& R) {
-  face_fields_seq<ORD, F0, DIR, STAGE_KIN>(P, c, L, R, std::make_integer_sequence<int, F1 - F0>());
+  face_fields_seq<ORD, F0, DIR, STAGE_KIN, ST>(P, c, L, R, std::make_integer_sequence<int, F1 - F0>());
 }
 
 // ---------------------------------------------------------------------------
@@ -162,13 +163,18 @@ template <typename T> __device__ inline T mcl_slope(T fa, T fb, int kind = 2) {
   return s * mn(mn(T(2) * fab(fa), T(2) * fab(fb)), T(0.5) * fab(fa + fb));
 }
 
-// left and right face values between the cells at c and c+st
-// (u_L = u_i + FAC mcl(.), u_R = u_{i+1} - FAC mcl(.), FAC = 0.5); the
-// half-slopes are returned too, for the "_m" states
-template <typename T>
-__device__ inline void mcl_rec(int slop, const double* __restrict__ a, int64_t c, int64_t st, T& l, T& r, T* u01 = nullptr,
+// left and right face values between cell c and its +x (DIR 0) or +y (DIR 1)
+// neighbour (u_L = u_i + FAC mcl(.), u_R = u_{i+1} - FAC mcl(.), FAC = 0.5);
+// the half-slopes are returned too, for the "_m" states
+template <int DIR, typename T, typename ST>
+__device__ inline void mcl_rec(int slop, const ST* __restrict__ a, const Cell& c, T& l, T& r, T* u01 = nullptr,
                                T* hs = nullptr) {
-  const T um = (T)a[c - st], u0 = (T)a[c], u1 = (T)a[c + st], u2 = (T)a[c + 2 * st];
+  T um, u0, u1, u2;
+  if constexpr (DIR == 0) {
+    um = (T)at_cell<-1>(a, c); u0 = (T)at_cell<0>(a, c); u1 = (T)at_cell<1>(a, c); u2 = (T)at_cell<2>(a, c);
+  } else {
+    um = (T)at_cell(a, c, -1); u0 = (T)at_cell(a, c); u1 = (T)at_cell(a, c, 1); u2 = (T)at_cell(a, c, 2);
+  }
   const T sl = T(0.5) * mcl_slope(u1 - u0, u0 - um, slop);
   const T sr = T(0.5) * mcl_slope(u2 - u1, u1 - u0, slop);
   l = u0 + sl;
@@ -212,29 +218,29 @@ template <typename T> __device__ inline T mcl_lf(T al, T ar, T ul, T ur) { retur
 
 // the fluxes of the face between the cells at c and c+st, DIR 0 = x (FX_*
 // slots), 1 = y (FY_* slots)
-template <int DIR, typename T>
-__device__ inline void mcl_face(const Planes& P, const Scheme& S, int64_t c, int64_t st, T* f) {
+template <int DIR, typename ST, typename T>
+__device__ inline void mcl_face(const Planes& P, const Scheme& S, const Cell& c, T* f) {
   McSide<T> L, R;
   T e0[2], es[2], b0[2], bs[2];  // cell values and half-slopes of the "_m" pair
-  mcl_rec(S.slop, P.s[S_PSI], c, st, L.psi, R.psi);
-  mcl_rec(S.slop, P.s[S_PHI], c, st, L.phi, R.phi);
-  mcl_rec(S.slop, P.s[S_EX], c, st, L.ex, R.ex, DIR == 1 ? e0 : (T*)nullptr, DIR == 1 ? es : (T*)nullptr);
-  mcl_rec(S.slop, P.s[S_EY], c, st, L.ey, R.ey);
-  mcl_rec(S.slop, P.s[S_EZ], c, st, L.ez, R.ez, DIR == 0 ? e0 : (T*)nullptr, DIR == 0 ? es : (T*)nullptr);
-  mcl_rec(S.slop, P.s[S_BX], c, st, L.bx, R.bx);
-  mcl_rec(S.slop, P.s[S_BY], c, st, L.by, R.by, DIR == 0 ? b0 : (T*)nullptr, DIR == 0 ? bs : (T*)nullptr);
-  mcl_rec(S.slop, P.s[S_BZ], c, st, L.bz, R.bz, DIR == 1 ? b0 : (T*)nullptr, DIR == 1 ? bs : (T*)nullptr);
-  mcl_rec(S.slop, P.s[S_Q], c, st, L.q, R.q);
-  mcl_rec(S.slop, P.s[S_D], c, st, L.d, R.d);
-  mcl_rec(S.slop, P.s[S_TAU], c, st, L.tau, R.tau);
-  mcl_rec(S.slop, P.s[S_SX], c, st, L.sx, R.sx);
-  mcl_rec(S.slop, P.s[S_SY], c, st, L.sy, R.sy);
-  mcl_rec(S.slop, P.s[S_SZ], c, st, L.sz, R.sz);
-  mcl_rec(S.slop, kin_plane(P, K_VX), c, st, L.vx, R.vx);
-  mcl_rec(S.slop, kin_plane(P, K_VY), c, st, L.vy, R.vy);
-  mcl_rec(S.slop, kin_plane(P, K_VZ), c, st, L.vz, R.vz);
-  mcl_rec(S.slop, kin_plane(P, K_P), c, st, L.p, R.p);
-  mcl_rec(S.slop, kin_plane(P, K_RHO), c, st, L.rho, R.rho);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_PSI), c, L.psi, R.psi);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_PHI), c, L.phi, R.phi);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_EX), c, L.ex, R.ex, DIR == 1 ? e0 : (T*)nullptr, DIR == 1 ? es : (T*)nullptr);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_EY), c, L.ey, R.ey);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_EZ), c, L.ez, R.ez, DIR == 0 ? e0 : (T*)nullptr, DIR == 0 ? es : (T*)nullptr);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_BX), c, L.bx, R.bx);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_BY), c, L.by, R.by, DIR == 0 ? b0 : (T*)nullptr, DIR == 0 ? bs : (T*)nullptr);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_BZ), c, L.bz, R.bz, DIR == 1 ? b0 : (T*)nullptr, DIR == 1 ? bs : (T*)nullptr);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_Q), c, L.q, R.q);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_D), c, L.d, R.d);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_TAU), c, L.tau, R.tau);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_SX), c, L.sx, R.sx);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_SY), c, L.sy, R.sy);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_SZ), c, L.sz, R.sz);
+  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_VX), c, L.vx, R.vx);
+  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_VY), c, L.vy, R.vy);
+  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_VZ), c, L.vz, R.vz);
+  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_P), c, L.p, R.p);
+  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_RHO), c, L.rho, R.rho);
   // "_m" states: the cell value negated, the slope kept
   // (16_hll_flow_mcl.f95:634-655, 708-737)
   const T em_l = (-e0[0]) + es[0], em_r = (-e0[1]) - es[1];
@@ -278,29 +284,29 @@ __device__ inline void mcl_face(const Planes& P, const Scheme& S, int64_t c, int
 // The face states of HLLC with the MC limiter (flux_solver = 4,
 // 16_hllc_flow_mcl.f95:1760-2479, the states and fluxes of hll_flow), as
 // the HLLC solve reads them
-template <int DIR, typename T>
-__device__ inline void mcl_sides(const Planes& P, const Scheme& S, int64_t c, int64_t st, Side<T>& L, Side<T>& R) {
+template <int DIR, typename ST, typename T>
+__device__ inline void mcl_sides(const Planes& P, const Scheme& S, const Cell& c, Side<T>& L, Side<T>& R) {
   McSide<T> l, r;
   T e0[2], es[2], b0[2], bs[2];
-  mcl_rec(S.slop, P.s[S_PSI], c, st, l.psi, r.psi);
-  mcl_rec(S.slop, P.s[S_PHI], c, st, l.phi, r.phi);
-  mcl_rec(S.slop, P.s[S_EX], c, st, l.ex, r.ex, DIR == 1 ? e0 : (T*)nullptr, DIR == 1 ? es : (T*)nullptr);
-  mcl_rec(S.slop, P.s[S_EY], c, st, l.ey, r.ey);
-  mcl_rec(S.slop, P.s[S_EZ], c, st, l.ez, r.ez, DIR == 0 ? e0 : (T*)nullptr, DIR == 0 ? es : (T*)nullptr);
-  mcl_rec(S.slop, P.s[S_BX], c, st, l.bx, r.bx);
-  mcl_rec(S.slop, P.s[S_BY], c, st, l.by, r.by, DIR == 0 ? b0 : (T*)nullptr, DIR == 0 ? bs : (T*)nullptr);
-  mcl_rec(S.slop, P.s[S_BZ], c, st, l.bz, r.bz, DIR == 1 ? b0 : (T*)nullptr, DIR == 1 ? bs : (T*)nullptr);
-  mcl_rec(S.slop, P.s[S_Q], c, st, l.q, r.q);
-  mcl_rec(S.slop, P.s[S_D], c, st, l.d, r.d);
-  mcl_rec(S.slop, P.s[S_TAU], c, st, l.tau, r.tau);
-  mcl_rec(S.slop, P.s[S_SX], c, st, l.sx, r.sx);
-  mcl_rec(S.slop, P.s[S_SY], c, st, l.sy, r.sy);
-  mcl_rec(S.slop, P.s[S_SZ], c, st, l.sz, r.sz);
-  mcl_rec(S.slop, kin_plane(P, K_VX), c, st, l.vx, r.vx);
-  mcl_rec(S.slop, kin_plane(P, K_VY), c, st, l.vy, r.vy);
-  mcl_rec(S.slop, kin_plane(P, K_VZ), c, st, l.vz, r.vz);
-  mcl_rec(S.slop, kin_plane(P, K_P), c, st, l.p, r.p);
-  mcl_rec(S.slop, kin_plane(P, K_RHO), c, st, l.rho, r.rho);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_PSI), c, l.psi, r.psi);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_PHI), c, l.phi, r.phi);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_EX), c, l.ex, r.ex, DIR == 1 ? e0 : (T*)nullptr, DIR == 1 ? es : (T*)nullptr);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_EY), c, l.ey, r.ey);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_EZ), c, l.ez, r.ez, DIR == 0 ? e0 : (T*)nullptr, DIR == 0 ? es : (T*)nullptr);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_BX), c, l.bx, r.bx);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_BY), c, l.by, r.by, DIR == 0 ? b0 : (T*)nullptr, DIR == 0 ? bs : (T*)nullptr);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_BZ), c, l.bz, r.bz, DIR == 1 ? b0 : (T*)nullptr, DIR == 1 ? bs : (T*)nullptr);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_Q), c, l.q, r.q);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_D), c, l.d, r.d);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_TAU), c, l.tau, r.tau);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_SX), c, l.sx, r.sx);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_SY), c, l.sy, r.sy);
+  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_SZ), c, l.sz, r.sz);
+  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_VX), c, l.vx, r.vx);
+  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_VY), c, l.vy, r.vy);
+  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_VZ), c, l.vz, r.vz);
+  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_P), c, l.p, r.p);
+  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_RHO), c, l.rho, r.rho);
   Side<T>* sd[2] = {&L, &R};
   const McSide<T>* ms[2] = {&l, &r};
 #pragma unroll
@@ -331,7 +337,7 @@ __device__ inline void mcl_sides(const Planes& P, const Scheme& S, int64_t c, in
 // ---------------------------------------------------------------------------
 // J, FD, Ftau, FS along DIR at cell (i,j) = k, with the t^n W and enthalpy
 // of startconvar (06_conserved_var.f95:92-109)
-template <int DIR, typename T>
+template <int DIR, typename ST, typename T>
 __device__ inline void lax_cell_fluxes(const Geom& g, const Planes& P, const Scheme& S, int i, int j, int64_t k,
                                        T* out) {
   if (i < 0 || i > g.imax || j < 0 || j > g.jmax) {
@@ -341,24 +347,24 @@ __device__ inline void lax_cell_fluxes(const Geom& g, const Planes& P, const Sch
   }
   // flowinit's cell fluxes: of v^n, p^n, rho^n, or with REC_PRIM = 1 of the
   // stage's primitives (14_flowinit.f95:376-489)
-  const T vx = (T)kin_plane(P, K_VX)[k], vy = (T)kin_plane(P, K_VY)[k], vz = (T)kin_plane(P, K_VZ)[k];
-  const T p = (T)kin_plane(P, K_P)[k], rho = (T)kin_plane(P, K_RHO)[k];
-  const T ex = (T)P.s[S_EX][k], ey = (T)P.s[S_EY][k], ez = (T)P.s[S_EZ][k];
-  const T bx = (T)P.s[S_BX][k], by = (T)P.s[S_BY][k], bz = (T)P.s[S_BZ][k];
+  const T vx = (T)kin_src<ST>(P, K_VX)[k], vy = (T)kin_src<ST>(P, K_VY)[k], vz = (T)kin_src<ST>(P, K_VZ)[k];
+  const T p = (T)kin_src<ST>(P, K_P)[k], rho = (T)kin_src<ST>(P, K_RHO)[k];
+  const T ex = (T)stage_src<ST>(P, S_EX)[k], ey = (T)stage_src<ST>(P, S_EY)[k], ez = (T)stage_src<ST>(P, S_EZ)[k];
+  const T bx = (T)stage_src<ST>(P, S_BX)[k], by = (T)stage_src<ST>(P, S_BY)[k], bz = (T)stage_src<ST>(P, S_BZ)[k];
   const T w = T(1) / sqrt(T(1) - ((sq(vx) + sq(vy)) + sq(vz)));
   const T eps = p / (((T)S.gamma - T(1)) * rho);
   const T h = rho * (T(1) + eps) + p;
   const T e2 = (sq(ex) + sq(ey)) + sq(ez), b2 = (sq(bx) + sq(by)) + sq(bz);
   const T hw2 = h * sq(w);
-  out[0] = (T)P.s[DIR == 0 ? S_JX : S_JY][k];
+  out[0] = (T)stage_src<ST>(P, DIR == 0 ? S_JX : S_JY)[k];
   if constexpr (DIR == 0) {
-    out[1] = (T)P.s[S_D][k] * vx;
+    out[1] = (T)stage_src<ST>(P, S_D)[k] * vx;
     out[2] = (bz * ey - by * ez) + hw2 * vx;
     out[3] = ((((-sq(ex)) - sq(bx)) + hw2 * sq(vx)) + T(0.5) * (e2 + b2)) + p;
     out[4] = ((-(ex * ey)) - bx * by) + (hw2 * vx) * vy;
     out[5] = ((-(ex * ez)) - bx * bz) + (hw2 * vx) * vz;
   } else {
-    out[1] = (T)P.s[S_D][k] * vy;
+    out[1] = (T)stage_src<ST>(P, S_D)[k] * vy;
     out[2] = (bx * ez - bz * ex) + hw2 * vy;
     out[3] = ((-(ex * ey)) - bx * by) + (hw2 * vx) * vy;
     out[4] = ((((-sq(ey)) - sq(by)) + hw2 * sq(vy)) + T(0.5) * (e2 + b2)) + p;
@@ -377,14 +383,14 @@ template <typename T> __device__ inline T lax_face_value(int slop, const T* a, c
   return T(0.5) * (l + r);
 }
 
-template <typename T> __device__ inline void lax_ld(const double* __restrict__ a, const int64_t* k, T* v) {
+template <typename T, typename ST> __device__ inline void lax_ld(const ST* __restrict__ a, const int64_t* k, T* v) {
 #pragma unroll
   for (int c = 0; c < 4; c++) v[c] = (T)a[k[c]];
 }
 
 // the fluxes of the face between cell (i,j) and its +x (DIR 0) or +y
 // (DIR 1) neighbour
-template <int DIR, typename T>
+template <int DIR, typename ST, typename T>
 __device__ inline void lax_face(const Geom& g, const Planes& P, const Scheme& S, int i, int j, T* f) {
   int64_t k[4];
   T fl[4][6];
@@ -392,12 +398,12 @@ __device__ inline void lax_face(const Geom& g, const Planes& P, const Scheme& S,
   for (int c = 0; c < 4; c++) {
     const int ii = DIR == 0 ? i + c - 1 : i, jj = DIR == 1 ? j + c - 1 : j;
     k[c] = g.at(ii, jj);
-    lax_cell_fluxes<DIR>(g, P, S, ii, jj, k[c], fl[c]);
+    lax_cell_fluxes<DIR, ST>(g, P, S, ii, jj, k[c], fl[c]);
   }
   T psi[4], phi[4], ex[4], ey[4], ez[4], bx[4], by[4], bz[4];
-  lax_ld(P.s[S_PSI], k, psi); lax_ld(P.s[S_PHI], k, phi);
-  lax_ld(P.s[S_EX], k, ex); lax_ld(P.s[S_EY], k, ey); lax_ld(P.s[S_EZ], k, ez);
-  lax_ld(P.s[S_BX], k, bx); lax_ld(P.s[S_BY], k, by); lax_ld(P.s[S_BZ], k, bz);
+  lax_ld(stage_src<ST>(P, S_PSI), k, psi); lax_ld(stage_src<ST>(P, S_PHI), k, phi);
+  lax_ld(stage_src<ST>(P, S_EX), k, ex); lax_ld(stage_src<ST>(P, S_EY), k, ey); lax_ld(stage_src<ST>(P, S_EZ), k, ez);
+  lax_ld(stage_src<ST>(P, S_BX), k, bx); lax_ld(stage_src<ST>(P, S_BY), k, by); lax_ld(stage_src<ST>(P, S_BZ), k, bz);
   if constexpr (DIR == 0) {  // 15_lax_flow.f95:930-1180
     f[FX_EXPSI] = lax_face_value(S.slop, ex, psi);
     f[FX_BXPHI] = lax_face_value(S.slop, bx, phi);
@@ -424,7 +430,7 @@ __device__ inline void lax_face(const Geom& g, const Planes& P, const Scheme& S,
     T a[4], u[4];
 #pragma unroll
     for (int c = 0; c < 4; c++) a[c] = fl[c][t];
-    lax_ld(P.s[us[t]], k, u);
+    lax_ld(stage_src<ST>(P, us[t]), k, u);
     f[FX_J + t] = lax_face_value(S.slop, a, u);
   }
 }
@@ -434,12 +440,13 @@ __device__ inline void lax_face(const Geom& g, const Planes& P, const Scheme& S,
 // array is dead after its put, which keeps the other solve's registers free
 // of it.  YFIRST solves the y face first (the two solves are independent
 // except under HLLE, whose y solve starts from the x solve's last iterate).
-template <int ORD, int SOLVER, typename T, bool YFIRST = false, bool STAGE_KIN = true, typename PutX, typename PutY>
+template <int ORD, int SOLVER, typename T, typename ST, bool YFIRST = false, bool STAGE_KIN = true, typename PutX,
+          typename PutY>
 __device__ __forceinline__ void face_pair(const Geom& g, const Planes& P, const Scheme& S, const StatusRef& st, int i,
                                           int j, PutX put_x, PutY put_y) {
   static_assert(!(YFIRST && SOLVER == 6), "the HLLE y solve needs the x solve first");
   const int64_t c = g.at(i, j);
-  const int64_t sx = 1, sy = g.pitch;
+  const Cell cc = cell_of(g, i, j);
   if constexpr (SOLVER == 3 || SOLVER == 4) {
     // HLLE / HLLC + MC limiter: x solve first (the y solve starts from its last iterate)
     T f[FX_N > FY_N ? FX_N : FY_N];
@@ -447,15 +454,15 @@ __device__ __forceinline__ void face_pair(const Geom& g, const Planes& P, const 
     T xseed = T(0), vlast = T(0);
     Side<T> sl, sr;
     if (seed) {
-      mcl_sides<1>(P, S, c, sy, sl, sr);
+      mcl_sides<1, ST>(P, S, cc, sl, sr);
       xseed = hlle_y_ery<T, true>(sl, sr);
     }
-    mcl_sides<0>(P, S, c, sx, sl, sr);
+    mcl_sides<0, ST>(P, S, cc, sl, sr);
     int code = SOLVER == 3 ? hlle_mcl_face<0>((T)S.gamma, sl, sr, f, seed, xseed, vlast)
                            : hllc_x<T, true>(sl, sr, f, seed, xseed, &vlast);
     if (code) report(st, code, i, j);
     put_x(f);
-    mcl_sides<1>(P, S, c, sy, sl, sr);
+    mcl_sides<1, ST>(P, S, cc, sl, sr);
     T unused;
     code = SOLVER == 3 ? hlle_mcl_face<1>((T)S.gamma, sl, sr, f, seed, vlast, unused)
                        : hllc_y<T, true>(sl, sr, f, seed, vlast);
@@ -467,8 +474,8 @@ __device__ __forceinline__ void face_pair(const Geom& g, const Planes& P, const 
     T f[FX_N > FY_N ? FX_N : FY_N];
     auto face = [&](auto dir) {
       constexpr int D = decltype(dir)::value;
-      if constexpr (SOLVER == 1) lax_face<D>(g, P, S, i, j, f);
-      else mcl_face<D>(P, S, c, D == 0 ? sx : sy, f);
+      if constexpr (SOLVER == 1) lax_face<D, ST>(g, P, S, i, j, f);
+      else mcl_face<D, ST>(P, S, cc, f);
       if constexpr (D == 0) put_x(f);
       else put_y(f);
     };
@@ -483,9 +490,8 @@ __device__ __forceinline__ void face_pair(const Geom& g, const Planes& P, const 
   }
   Side<T> xl, xr, yl, yr;
   // kinematics of both faces first: the fallbacks couple them
-  const Cell cc = cell_of(g, i, j);
-  face_fields<ORD, F_VX, F_PSI, 0, STAGE_KIN>(P, cc, xl, xr);
-  face_fields<ORD, F_VX, F_PSI, 1, STAGE_KIN>(P, cc, yl, yr);
+  face_fields<ORD, F_VX, F_PSI, 0, STAGE_KIN, ST>(P, cc, xl, xr);
+  face_fields<ORD, F_VX, F_PSI, 1, STAGE_KIN, ST>(P, cc, yl, yr);
   // superluminal fallback, 16_hll_flow_mpx.f95:1392-1461 (same in hllc;
   // hlle only prints, 16_hlle_flow_mpx.f95:2270-2300)
   if (SOLVER != 6) {
@@ -502,25 +508,27 @@ __device__ __forceinline__ void face_pair(const Geom& g, const Planes& P, const 
     }
   }
   if (SOLVER == 7) {  // density fix-up, 16_hllc_flow_mpx.f95:2663-2693
-    T rc = (T)(0.1 * P.p[P_RHO][c]);
-    if (yl.rho < 0.0) yl.rho = rc;
-    else if (yr.rho < 0.0) yr.rho = rc;
-    else if (xl.rho < 0.0) xl.rho = rc;
-    else if (xr.rho < 0.0) xr.rho = rc;
+    if (yl.rho < T(0) || yr.rho < T(0) || xl.rho < T(0) || xr.rho < T(0)) {
+      T rc = (T)(0.1 * P.p[P_RHO][c]);
+      if (yl.rho < T(0)) yl.rho = rc;
+      else if (yr.rho < T(0)) yr.rho = rc;
+      else if (xl.rho < T(0)) xl.rho = rc;
+      else xr.rho = rc;
+    }
   }
   constexpr bool HW = SOLVER == 6;
   // HLLE: first Newton point of the x contact solve in the reference build
   // is the y face's (E x B)_y; that of the y solve is the x solve's last iterate
   T seed_x = T(0), seed_y = T(0);
   if (SOLVER == 6 && S.hllc_seed_ref) {
-    face_fields<ORD, F_EX, F_EX + 1, 1, STAGE_KIN>(P, cc, yl, yr);
-    face_fields<ORD, F_EZ, F_EZ + 1, 1, STAGE_KIN>(P, cc, yl, yr);
-    face_fields<ORD, F_BX, F_BX + 1, 1, STAGE_KIN>(P, cc, yl, yr);
-    face_fields<ORD, F_BZ, F_BZ + 1, 1, STAGE_KIN>(P, cc, yl, yr);
+    face_fields<ORD, F_EX, F_EX + 1, 1, STAGE_KIN, ST>(P, cc, yl, yr);
+    face_fields<ORD, F_EZ, F_EZ + 1, 1, STAGE_KIN, ST>(P, cc, yl, yr);
+    face_fields<ORD, F_BX, F_BX + 1, 1, STAGE_KIN, ST>(P, cc, yl, yr);
+    face_fields<ORD, F_BZ, F_BZ + 1, 1, STAGE_KIN, ST>(P, cc, yl, yr);
     seed_x = hlle_y_ery(yl, yr);
   }
   auto xface = [&]() {
-    face_fields<ORD, F_PSI, F_NQ, 0, STAGE_KIN>(P, cc, xl, xr);
+    face_fields<ORD, F_PSI, F_NQ, 0, STAGE_KIN, ST>(P, cc, xl, xr);
     side_physics<0, HW>((T)S.gamma, xl);
     side_physics<0, HW>((T)S.gamma, xr);
     T f[FX_N];
@@ -536,7 +544,7 @@ __device__ __forceinline__ void face_pair(const Geom& g, const Planes& P, const 
     put_x(f);
   };
   auto yface = [&]() {
-    face_fields<ORD, F_PSI, F_NQ, 1, STAGE_KIN>(P, cc, yl, yr);
+    face_fields<ORD, F_PSI, F_NQ, 1, STAGE_KIN, ST>(P, cc, yl, yr);
     side_physics<1, HW>((T)S.gamma, yl);
     side_physics<1, HW>((T)S.gamma, yr);
     T f[FY_N];
@@ -589,7 +597,7 @@ k_faces(Geom g, Planes P, Scheme S, StatusRef st) {
   const int j = by * blockDim.y + threadIdx.y - 1;
   if (i > g.imax || j > g.jmax) return;
   const int64_t c = g.at(i, j);
-  face_pair<ORD, SOLVER, T>(
+  face_pair<ORD, SOLVER, T, double>(
       g, P, S, st, i, j,
       [&](const T* f) {
 #pragma unroll
@@ -658,9 +666,7 @@ static_assert(offsetof(MarchArgs, P) == 0, "argument block layout");
 //     2-12 VGPRs and runs 36 % faster, HLLE (one y-row buffer, below) 36 %,
 //     Lax-Friedrichs 32 %, the MCL solvers (63-114 spilled) 17-20 %;
 //   FP32: 3.  With the stencils loaded ahead, 4 waves (128 VGPRs) spill
-//     22-37 VGPRs under HLLC and ran 7 % slower (HLLE 13 %), 2 the same; the
-//     MCL solvers' 178-192 VGPRs ran 2 waves per SIMD unbounded and 9-19 %
-//     slower.
+//     and ran 3-6 % slower under HLLC, HLLE and HLL, 19 % under HLL + MC.
 template <typename T, int SOLVER>
 constexpr int march_min_waves() {
   if constexpr (sizeof(T) == 8) return CUEVA_MARCH_F64_WAVES > 0 ? CUEVA_MARCH_F64_WAVES : 2;
@@ -739,7 +745,7 @@ k_faces_march(MarchArgs args) {
       }
     };
     if (face_ok) {
-      face_pair<ORD, SOLVER, T, !XLDS, false>(g, P, S, st, i, j, put_x, put_y);
+      face_pair<ORD, SOLVER, T, T, !XLDS, false>(g, P, S, st, i, j, put_x, put_y);
     } else {
       T z[FX_N > FY_N ? FX_N : FY_N];
 #pragma unroll
@@ -769,7 +775,8 @@ k_faces_march(MarchArgs args) {
         dfy[a] = ddy<T>(S, fyb[b][w][a][lane] - below);
       }
       const int64_t k = g.at(i, j);
-      const Rhs r = rhs_of<T, false>(P, S, k, dfx, dfy);  // never with REC_PRIM = 1
+      // never with REC_PRIM = 1
+      const Rhs r = rhs_of<T, false>(P, S, k, dfx, dfy, sizeof(T) == 4 && l == 0);
       if constexpr (!FINAL) {
         put_planes<R_N>(P.rhs[l], k, r.r, S.stream > 0);
         // the next stage's state of this point (pointwise in U^n and the
@@ -778,7 +785,7 @@ k_faces_march(MarchArgs args) {
         stage_point(P, S, l + 1, k, false, P.p[P_VX][k], P.p[P_VY][k], P.p[P_VZ][k], P.p[P_EX][k], P.p[P_EY][k],
                     P.p[P_EZ][k], P.p[P_BX][k], P.p[P_BY][k], P.p[P_BZ][k], P.p[P_RHO][k], P.p[P_P][k],
                     P.p[P_PSI][k], P.p[P_PHI][k], P.p[P_Q][k], sv, &r);
-        store_stage(P.sn, k, sv, S.stream > 0);
+        store_stage<sizeof(T) == 4>(P.sn, P.snf, k, sv, false, S.full != 0, S.stream > 0);
       } else {
         double nu[A_N];
         final_update_from(P, S, k, r, nu);

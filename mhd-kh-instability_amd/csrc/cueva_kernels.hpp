@@ -22,7 +22,26 @@ struct PlaneList {
   double* a[32];
   int n;
   int nzero;  // the last nzero planes get 0 at every ghost point instead of a copy
+  float* f[24];  // FP32 planes, after the FP64 ones; the last nfzero get 0
+  int nf;
+  int nfzero;
 };
+// blocks in y of a k_fill_ghosts launch
+constexpr int GHOST_PLANES = 4;
+inline unsigned ghost_groups(const PlaneList& pl) {
+  return (unsigned)((pl.n + GHOST_PLANES - 1) / GHOST_PLANES + (pl.nf + GHOST_PLANES - 1) / GHOST_PLANES);
+}
+
+template <typename ST>
+__device__ inline void copy_ghosts(ST* const* a, int n, int nzero, int k0, int64_t src, int64_t dst) {
+  ST v[GHOST_PLANES];
+#pragma unroll
+  for (int k = 0; k < GHOST_PLANES; k++)
+    if (k0 + k < n) v[k] = k0 + k < n - nzero ? a[k0 + k][src] : ST(0);
+#pragma unroll
+  for (int k = 0; k < GHOST_PLANES; k++)
+    if (k0 + k < n) a[k0 + k][dst] = v[k];
+}
 
 // One thread copies one ghost point of GHOST_PLANES planes (blockIdx.y picks
 // them), their loads in flight together.  The fill is bound by latency: a
@@ -30,7 +49,6 @@ struct PlaneList {
 // time and took 14 us at 32x64, 21 at 128x256 and 36 at 2048x4096; now
 // 6.5, 6.6 and 21 us.  The bands left and right are walked row by row, 12
 // points each, so that neighbouring threads share cache lines.
-constexpr int GHOST_PLANES = 4;
 __global__ void __launch_bounds__(256) k_fill_ghosts(Geom g, PlaneList pl, StatusRef sr) {
   if (halted(sr)) return;
   const int im = g.imax, jm = g.jmax;
@@ -50,14 +68,9 @@ __global__ void __launch_bounds__(256) k_fill_ghosts(Geom g, PlaneList pl, Statu
   }
   const int64_t dst = g.at(i, j);
   const int64_t src = g.at(src_index(i, im, g.bcx), src_index(j, jm, g.bcy));
-  const int k0 = (int)blockIdx.y * GHOST_PLANES;
-  double v[GHOST_PLANES];
-#pragma unroll
-  for (int k = 0; k < GHOST_PLANES; k++)
-    if (k0 + k < pl.n) v[k] = k0 + k < pl.n - pl.nzero ? pl.a[k0 + k][src] : 0.0;
-#pragma unroll
-  for (int k = 0; k < GHOST_PLANES; k++)
-    if (k0 + k < pl.n) pl.a[k0 + k][dst] = v[k];
+  const int q = (int)blockIdx.y, nd = (pl.n + GHOST_PLANES - 1) / GHOST_PLANES;
+  if (q < nd) copy_ghosts(pl.a, pl.n, pl.nzero, q * GHOST_PLANES, src, dst);
+  else copy_ghosts(pl.f, pl.nf, pl.nfzero, (q - nd) * GHOST_PLANES, src, dst);
 }
 
 // at most 12 (65536 + 13) + 12 (65536 + 1): fits 32 bits
@@ -410,7 +423,9 @@ __global__ void k_stage_fused(Geom g, Planes P, Scheme S, int l, int halo, Statu
   stage_point(P, S, l, ks, ghost, P.p[P_VX][ks], P.p[P_VY][ks], P.p[P_VZ][ks], P.p[P_EX][ks], P.p[P_EY][ks],
               P.p[P_EZ][ks], P.p[P_BX][ks], P.p[P_BY][ks], P.p[P_BZ][ks], P.p[P_RHO][ks], P.p[P_P][ks],
               P.p[P_PSI][ks], P.p[P_PHI][ks], P.p[P_Q][ks], out);
-  store_stage(P.s, k, out);
+  store_stage(P.s, P.sf, k, out, l == 0, S.full != 0, false);
+  if (P.kf[0])
+    store_kin(P.kf, k, P.p[P_VX][ks], P.p[P_VY][ks], P.p[P_VZ][ks], P.p[P_P][ks], P.p[P_RHO][ks], false);
 }
 
 // Last stage right-hand side, sumfin, varfin and electricfield at one

@@ -19,17 +19,18 @@ struct Rhs { double r[R_N]; };
 // at 1024x2048 1.20 against 1.24.  Small grids, whose planes the 256 MB
 // Infinity Cache keeps from launch to launch, lose by it (HLL + MC at 300x700
 // 201 against 186 us).
-template <int N> __device__ inline void put_planes(double* const* p, int64_t k, const double* v, bool stream) {
+template <int N, typename ST>
+__device__ inline void put_planes(ST* const* p, int64_t k, const double* v, bool stream) {
   if (stream) {
     // the empty statements keep the compiler from merging the two branches'
     // stores into one that is not streamed
     asm volatile("");
 #pragma unroll
-    for (int t = 0; t < N; t++) __builtin_nontemporal_store(v[t], &p[t][k]);
+    for (int t = 0; t < N; t++) __builtin_nontemporal_store((ST)v[t], &p[t][k]);
     asm volatile("");
   } else {
 #pragma unroll
-    for (int t = 0; t < N; t++) p[t][k] = v[t];
+    for (int t = 0; t < N; t++) p[t][k] = (ST)v[t];
   }
 }
 
@@ -44,8 +45,12 @@ template <typename FT> __device__ inline FT ddy(const Scheme& S, FT a) {
 // dfx[a] = (Fx(i+1/2) - Fx(i-1/2))/dx and dfy likewise, formed in the flux
 // arithmetic FT (held in FT until used: a float difference widens exactly),
 // combined with the FP64 sources of the stage state.
+// from_prims (mixed marching step, first stage): psi phi B q from the primitive
+// planes, whose values the first stage's are (x + 0.0: a negative zero becomes
+// the positive one of un + dt 0)
 template <typename FT, bool STAGE_KIN = true>
-__device__ inline Rhs rhs_of(const Planes& P, const Scheme& S, int64_t k, const FT* dfx, const FT* dfy) {
+__device__ inline Rhs rhs_of(const Planes& P, const Scheme& S, int64_t k, const FT* dfx, const FT* dfy,
+                             bool from_prims = false) {
 #pragma clang fp contract(off)  // FP64: as the reference build, also inside the FP32 face unit
 #define DX(a) ((double)dfx[a])
 #define DY(a) ((double)dfy[a])
@@ -54,10 +59,14 @@ __device__ inline Rhs rhs_of(const Planes& P, const Scheme& S, int64_t k, const 
   double vx = kin_plane<STAGE_KIN>(P, K_VX)[k], vy = kin_plane<STAGE_KIN>(P, K_VY)[k],
          vz = kin_plane<STAGE_KIN>(P, K_VZ)[k];
   double w = 1.0 / sqrt(1.0 - ((sq(vx) + sq(vy)) + sq(vz)));
-  double q = P.s[S_Q][k];
+  const double* const* from = from_prims ? P.p : P.s;
+  static_assert((int)S_PSI == (int)P_PSI && (int)S_PHI == (int)P_PHI && (int)S_BX == (int)P_BX &&
+                    (int)S_BY == (int)P_BY && (int)S_BZ == (int)P_BZ, "same place in both plane sets");
+  const double q = (from_prims ? P.p[P_Q] : P.s[S_Q])[k] + 0.0, psi = from[S_PSI][k] + 0.0, phi = from[S_PHI][k] + 0.0;
+  const double bx = from[S_BX][k] + 0.0, by = from[S_BY][k] + 0.0, bz = from[S_BZ][k] + 0.0;
   Rhs o;
-  o.r[0] = ((((-DX(FX_EXPSI)) - DY(FY_EYPSI)) - 0.0) + q) - S.kpsi * P.s[S_PSI][k];
-  o.r[1] = (((-DX(FX_BXPHI)) - DY(FY_BYPHI)) - 0.0) - S.kphi * P.s[S_PHI][k];
+  o.r[0] = ((((-DX(FX_EXPSI)) - DY(FY_EYPSI)) - 0.0) + q) - S.kpsi * psi;
+  o.r[1] = (((-DX(FX_BXPHI)) - DY(FY_BYPHI)) - 0.0) - S.kphi * phi;
   o.r[2] = ((-DY(FY_EZBX)) + 0.0) - DX(FX_PHIBX);
   o.r[3] = ((-0.0) + DX(FX_EZBY)) - DY(FY_PHIBY);
   o.r[4] = ((-DX(FX_EYBZ)) + DY(FY_EXBZ)) - 0.0;
@@ -72,8 +81,8 @@ __device__ inline Rhs rhs_of(const Planes& P, const Scheme& S, int64_t k, const 
   o.r[13] = ((-DX(FX_FSZ)) - DY(FY_FSZ)) - 0.0;
 #undef DX
 #undef DY
-  ohm_source(S.sigma, w, vx, vy, vz, P.s[S_EX][k], P.s[S_EY][k], P.s[S_EZ][k], P.s[S_BX][k], P.s[S_BY][k],
-             P.s[S_BZ][k], o.r[R_SEX], o.r[R_SEY], o.r[R_SEZ]);
+  ohm_source(S.sigma, w, vx, vy, vz, P.s[S_EX][k], P.s[S_EY][k], P.s[S_EZ][k], bx, by, bz, o.r[R_SEX], o.r[R_SEY],
+             o.r[R_SEZ]);
   return o;
 }
 
@@ -239,10 +248,45 @@ __device__ inline void stage_point(const Planes& P, const Scheme& S, int l, int6
   out[S_JX] = jx; out[S_JY] = jy; out[S_JZ] = jz;
 }
 
-__device__ inline void store_stage(double* const* s, int64_t k, const double* v, bool stream = false) {
-  static_assert(S_EXA == 5 && S_EZA == 7, "the unused E* planes are 5 to 7");
-  put_planes<S_EXA>(s, k, v, stream);
-  put_planes<S_N - S_EZA - 1>(s + S_EZA + 1, k, v + S_EZA + 1, stream);
+// The stage state of one point, to the planes s and, with NARROW, the FP32
+// copies sf that the mixed form's stencils read.  What nothing reads is stored
+// only where `full` asks for it (the state that stays after the call): J_z;
+// and with NARROW D tau S J in FP64, which the stencils alone read, and the
+// first stage's psi phi B q in FP64, which are those of the primitive planes
+// (rhs_of takes them there).
+template <bool NARROW>
+__device__ inline void store_stage(double* const* s, float* const* sf, int64_t k, const double* v, bool first,
+                                   bool full, bool stream) {
+  static_assert(S_EXA == 5 && S_Q == 8 && S_EX == 14 && S_JX == 17 && S_N == 20, "plane order");
+  if (NARROW) {
+    put_planes<S_EXA>(sf, k, v, false);
+    put_planes<S_JZ - S_Q>(sf + S_Q, k, v + S_Q, false);
+    put_planes<3>(s + S_EX, k, v + S_EX, stream);
+    if (!first || full) {
+      put_planes<S_EXA>(s, k, v, stream);
+      put_planes<1>(s + S_Q, k, v + S_Q, stream);
+    }
+    if (full) {
+      put_planes<5>(s + S_D, k, v + S_D, stream);
+      put_planes<3>(s + S_JX, k, v + S_JX, stream);
+    }
+  } else {
+    put_planes<S_EXA>(s, k, v, stream);
+    put_planes<S_JZ - S_Q>(s + S_Q, k, v + S_Q, stream);
+    if (full) put_planes<1>(s + S_JZ, k, v + S_JZ, stream);
+  }
+}
+// the same where the form is not known at compile time
+__device__ inline void store_stage(double* const* s, float* const* sf, int64_t k, const double* v, bool first,
+                                   bool full, bool stream) {
+  if (sf[0]) store_stage<true>(s, sf, k, v, first, full, stream);
+  else store_stage<false>(s, sf, k, v, first, full, stream);
+}
+__device__ inline void store_kin(float* const* kf, int64_t k, double vx, double vy, double vz, double p, double rho,
+                                 bool stream) {
+  static_assert(K_VX == 0 && K_VY == 1 && K_VZ == 2 && K_P == 3 && K_RHO == 4, "plane order");
+  const double v[K_N] = {vx, vy, vz, p, rho};
+  put_planes<K_N>(kf, k, v, false);
 }
 
 // primitive recovery of one point (Cardano, 12_varprimitive.f95) and the
@@ -301,7 +345,8 @@ __device__ inline void recover_point(const Planes& P, const Scheme& S, const Sta
     double sv[S_N];
     stage_point(P, S, 0, k, false, o.vx, o.vy, o.vz, in.ex, in.ey, in.ez, in.bx, in.by, in.bz, o.rho, o.p,
                 nu[A_PSI], nu[A_PHI], nu[A_Q], sv);
-    store_stage(P.sn, k, sv, S.stream > 0);
+    store_stage(P.sn, P.snf, k, sv, true, S.full != 0, S.stream > 0);
+    if (P.knf[0]) store_kin(P.knf, k, o.vx, o.vy, o.vz, o.p, o.rho, S.stream > 0);
   }
 }
 
@@ -311,7 +356,8 @@ __device__ inline void stage0_after_c2p(Planes& P, const Scheme& S, int64_t k, c
   double out[S_N];
   stage_point(P, S, 0, k, false, o.vx, o.vy, o.vz, in.ex, in.ey, in.ez, in.bx, in.by, in.bz, o.rho, o.p,
               P.p[P_PSI][k], P.p[P_PHI][k], P.p[P_Q][k], out);
-  store_stage(P.s, k, out, S.stream > 1);
+  store_stage(P.s, P.sf, k, out, true, S.full != 0, S.stream > 1);
+  if (P.knf[0]) store_kin(P.knf, k, o.vx, o.vy, o.vz, o.p, o.rho, S.stream > 1);
 }
 
 }  // namespace cueva
