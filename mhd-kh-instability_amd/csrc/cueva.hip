@@ -265,7 +265,7 @@ extern "C" int cueva_create(const cueva_params* p, cueva_ctx** out) {
   Geom& g = c->g;
   g.imax = p->imax;
   g.jmax = p->jmax;
-  g.pitch = ((p->imax + 16) + 7) / 8 * 8;
+  g.pitch = (X0 + p->imax + 7 + 15) / 16 * 16;
   g.rows = p->jmax + 13;
   g.plane = ((int64_t)g.pitch * g.rows + 63) / 64 * 64;
   g.bcx = p->bc_x;
@@ -561,9 +561,9 @@ static int copy_planes_strided(cueva_ctx* c, double* const* planes, int n, doubl
     double* h = host + (size_t)k * hw * hh;
     const size_t pitch = (size_t)g.pitch * sizeof(double);
     if (up)
-      HIPCHK(hipMemcpy2DAsync(planes[k] + 2, pitch, h, row, row, hh, hipMemcpyHostToDevice, c->stream));
+      HIPCHK(hipMemcpy2DAsync(planes[k] + (X0 - GH), pitch, h, row, row, hh, hipMemcpyHostToDevice, c->stream));
     else
-      HIPCHK(hipMemcpy2DAsync(h, row, planes[k] + 2, pitch, row, hh, hipMemcpyDeviceToHost, c->stream));
+      HIPCHK(hipMemcpy2DAsync(h, row, planes[k] + (X0 - GH), pitch, row, hh, hipMemcpyDeviceToHost, c->stream));
   }
   return CUEVA_OK;
 }
@@ -1555,7 +1555,7 @@ extern "C" int cueva_reduce_globals_noalloc(const cueva_params* p, const double*
   double* partial = scratch_of(dev);
   if (!partial) return CUEVA_E_HIP;
   // the caller's planes in the host layout (-6:imax+6, -6:jmax+6), x fastest:
-  // with pitch imax+13, Geom::at(i, j) - 2 is the element's index in a plane
+  // with pitch imax+13, Geom::at(i, j) - (X0 - 6) is the element's index in a plane
   Geom g;
   memset(&g, 0, sizeof(g));
   g.imax = p->imax;
@@ -1567,8 +1567,8 @@ extern "C" int cueva_reduce_globals_noalloc(const cueva_params* p, const double*
   g.bcy = p->bc_y;
   Planes P;
   memset(&P, 0, sizeof(P));
-  for (int k = 0; k < P_N; k++) P.p[k] = (double*)(prims14 + (size_t)k * (size_t)g.plane) - 2;
-  for (int k = 0; k < 5; k++) P.c[k] = (double*)(cons5 + (size_t)k * (size_t)g.plane) - 2;
+  for (int k = 0; k < P_N; k++) P.p[k] = (double*)(prims14 + (size_t)k * (size_t)g.plane) - (X0 - GH);
+  for (int k = 0; k < 5; k++) P.c[k] = (double*)(cons5 + (size_t)k * (size_t)g.plane) - (X0 - GH);
   Scheme S;
   memset(&S, 0, sizeof(S));
   double d[5];

@@ -15,19 +15,27 @@
 namespace cueva {
 
 constexpr int GH = 6;  // ghost layers (scalar.f95:9)
+// Elements before column 0 in a row.  With a pitch of a multiple of 16, column
+// 0 of every row starts a 128-byte cache line of an FP64 plane (half a line of
+// the FP32 copies), so that a wavefront of the pointwise kernels, which take
+// columns from a multiple of 64 on, moves whole lines: recovery pass at
+// 2048x4096 0.535 -> 0.509 ms, mixed + learned 0.602 -> 0.516, HLLE mixed at
+// 1024x2048 0.147 -> 0.128 (32, whole FP32 lines too, measured the same there
+// and 0.3 % slower per step).
+constexpr int X0 = 16;
 
 // ---------------------------------------------------------------------------
 // grid geometry: plane of doubles with reference indices (-6:imax+6,-6:jmax+6)
 // ---------------------------------------------------------------------------
 struct Geom {
   int imax, jmax;
-  int pitch;         // doubles per row (>= imax+15, multiple of 8)
+  int pitch;         // doubles per row (>= X0+imax+7, multiple of 16)
   int rows;          // jmax + 13
   int64_t plane;     // doubles per plane (multiple of 64)
   int bcx, bcy;      // 0 copy, 1 periodic
-  // element (i,j) lives at offset (j+6)*pitch + (i+8)
+  // element (i,j) lives at offset (j+6)*pitch + (i+X0)
   __host__ __device__ inline int64_t at(int i, int j) const {
-    return (int64_t)(j + GH) * pitch + (i + 8);
+    return (int64_t)(j + GH) * pitch + (i + X0);
   }
 };
 

@@ -64,7 +64,7 @@ struct Cell {
   int pitch;
 };
 __device__ inline Cell cell_of(const Geom& g, int i, int j) {
-  return {(uint32_t)(i + 8) * 8u, (int64_t)(__builtin_amdgcn_readfirstlane(j) + GH) * g.pitch, g.pitch};
+  return {(uint32_t)(i + X0) * 8u, (int64_t)(__builtin_amdgcn_readfirstlane(j) + GH) * g.pitch, g.pitch};
 }
 // element (i + DI, j + dj)
 template <int DI = 0, typename ST> __device__ inline ST at_cell(const ST* __restrict__ a, const Cell& c, int dj = 0) {

@@ -86,7 +86,7 @@ __global__ void __launch_bounds__(256) k_rows_to_planes(const double* __restrict
   if (r >= rows) return;
   const int p = (r0 + r) / hh, j = (r0 + r) - p * hh, x = (int)(blockIdx.x * 256 + threadIdx.x);
   const double* s = buf + (int64_t)r * w;
-  double* d = pl.a[p] + (int64_t)j * pitch + 2;
+  double* d = pl.a[p] + (int64_t)j * pitch + (X0 - GH);
   double v[4];
 #pragma unroll
   for (int k = 0; k < 4; k++)
@@ -100,7 +100,7 @@ __global__ void __launch_bounds__(256) k_planes_to_rows(double* __restrict__ buf
   const int r = (int)(blockIdx.y * 4 + threadIdx.y);
   if (r >= rows) return;
   const int p = (r0 + r) / hh, j = (r0 + r) - p * hh, x = (int)(blockIdx.x * 256 + threadIdx.x);
-  const double* s = pl.a[p] + (int64_t)j * pitch + 2;
+  const double* s = pl.a[p] + (int64_t)j * pitch + (X0 - GH);
   double* d = buf + (int64_t)r * w;
   double v[4];
 #pragma unroll
