@@ -72,12 +72,13 @@ template <int DI = 0, typename ST> __device__ inline ST at_cell(const ST* __rest
   return *(const ST*)(row + (sizeof(ST) == 8 ? c.vo : c.vo >> 1) + DI * (int)sizeof(ST));
 }
 
-// the 2K+2 values of one quantity across the face, as loaded
-template <int ORD, typename ST> struct Sten { ST v[2 * MPc<ORD>::K + 2]; };
-template <int ORD, int DIR, typename ST, int... T>
-__device__ inline void sten_load(const ST* __restrict__ a, const Cell& c, Sten<ORD, ST>& s,
+// the NV values of one quantity across the face, as loaded (MPx: 2K+2; MC
+// limiter: 4)
+template <int NV, typename ST> struct Sten { ST v[NV]; };
+template <int DIR, typename ST, int... T>
+__device__ inline void sten_load(const ST* __restrict__ a, const Cell& c, Sten<(int)sizeof...(T), ST>& s,
                                  std::integer_sequence<int, T...>) {
-  constexpr int K = MPc<ORD>::K;
+  constexpr int K = (int)sizeof...(T) / 2 - 1;
   ((s.v[T] = DIR == 0 ? at_cell<DIR == 0 ? T - K : 0>(a, c) : at_cell(a, c, T - K)), ...);
 }
 
@@ -104,14 +105,12 @@ template <int F, typename T> __device__ inline T& face_slot(Side<T>& o) {
   return o.*m[F];
 }
 
-template <int ORD, int F, int DIR, bool STAGE_KIN, typename ST>
-__device__ inline void face_load(const Planes& P, const Cell& c, Sten<ORD, ST>& s) {
-  sten_load<ORD, DIR>(face_plane<F, DIR, STAGE_KIN, ST>(P), c, s,
-                      std::make_integer_sequence<int, 2 * MPc<ORD>::K + 2>());
+template <int F, int DIR, bool STAGE_KIN, int NV, typename ST>
+__device__ inline void face_load(const Planes& P, const Cell& c, Sten<NV, ST>& s) {
+  sten_load<DIR>(face_plane<F, DIR, STAGE_KIN, ST>(P), c, s, std::make_integer_sequence<int, NV>());
 }
-template <int ORD, int F, typename ST, typename T>
-__device__ inline void face_take(const Sten<ORD, ST>& s, Side<T>& L, Side<T>& R) {
-  constexpr int N = 2 * MPc<ORD>::K + 2;
+template <int ORD, int F, int N, typename ST, typename T>
+__device__ inline void face_take(const Sten<N, ST>& s, Side<T>& L, Side<T>& R) {
   T v[N];
 #pragma unroll
   for (int t = 0; t < N; t++) v[t] = (T)s.v[t];
@@ -127,13 +126,13 @@ template <int ORD, int F0, int DIR, bool STAGE_KIN, typename ST, typename T, int
 __device__ inline void face_fields_seq(const Planes& P, const Cell& c, Side<T>& L, Side<T>& R,
                                        std::integer_sequence<int, S...>) {
   constexpr int N = sizeof...(S), AH = face_ahead<ST>();
-  Sten<ORD, ST> b[AH + 1];
+  Sten<2 * MPc<ORD>::K + 2, ST> b[AH + 1];
   auto pre = [&](auto t) {
-    if constexpr (t() < AH && t() < N) face_load<ORD, F0 + t(), DIR, STAGE_KIN>(P, c, b[t()]);
+    if constexpr (t() < AH && t() < N) face_load<F0 + t(), DIR, STAGE_KIN>(P, c, b[t()]);
   };
   auto one = [&](auto t) {
     if constexpr (t() + AH < N)
-      face_load<ORD, F0 + t() + AH, DIR, STAGE_KIN>(P, c, b[(t() + AH) % (AH + 1)]);
+      face_load<F0 + t() + AH, DIR, STAGE_KIN>(P, c, b[(t() + AH) % (AH + 1)]);
     face_take<ORD, F0 + t()>(b[t() % (AH + 1)], L, R);
   };
   (pre(std::integral_constant<int, S>()), ...);
@@ -160,36 +159,14 @@ template <typename T> __device__ inline T mcl_slope(T fa, T fb, int kind = 2) {
   const T s = T(0.5) * (csign(fa) + csign(fb));
   if (kind == 1) return s * mn(fab(fa), fab(fb));
   if (kind == 3) return s * mn(mn(T(2) * fab(fa), T(2) * fab(fb)), mx(fab(fa), fab(fb)));
-  return s * mn(mn(T(2) * fab(fa), T(2) * fab(fb)), T(0.5) * fab(fa + fb));
+  // a NaN operand that FP64's minimum drops is NaN in the sum as well
+  return s * mn(T(2) * lim_mn(fab(fa), fab(fb)), T(0.5) * fab(fa + fb));
 }
-
-// left and right face values between cell c and its +x (DIR 0) or +y (DIR 1)
-// neighbour (u_L = u_i + FAC mcl(.), u_R = u_{i+1} - FAC mcl(.), FAC = 0.5);
-// the half-slopes are returned too, for the "_m" states
-template <int DIR, typename T, typename ST>
-__device__ inline void mcl_rec(int slop, const ST* __restrict__ a, const Cell& c, T& l, T& r, T* u01 = nullptr,
-                               T* hs = nullptr) {
-  T um, u0, u1, u2;
-  if constexpr (DIR == 0) {
-    um = (T)at_cell<-1>(a, c); u0 = (T)at_cell<0>(a, c); u1 = (T)at_cell<1>(a, c); u2 = (T)at_cell<2>(a, c);
-  } else {
-    um = (T)at_cell(a, c, -1); u0 = (T)at_cell(a, c); u1 = (T)at_cell(a, c, 1); u2 = (T)at_cell(a, c, 2);
-  }
-  const T sl = T(0.5) * mcl_slope(u1 - u0, u0 - um, slop);
-  const T sr = T(0.5) * mcl_slope(u2 - u1, u1 - u0, slop);
-  l = u0 + sl;
-  r = u1 - sr;
-  if (u01) { u01[0] = u0; u01[1] = u1; hs[0] = sl; hs[1] = sr; }
-}
-
-template <typename T> struct McSide { T psi, phi, ex, ey, ez, bx, by, bz, q, d, tau, sx, sy, sz, vx, vy, vz, p, rho; };
 
 // J, FD, Ftau and the three FS of one side: E^2+B^2 (16_hll_flow_mcl.f95:821),
 // W (:900), E.v (:995), J (:1033), FD (:1050), eps and h (:1124), Ftau
 // (:1181), FS (:1198-1241)
-template <int DIR, typename T>
-__device__ inline void mcl_side_fluxes(T gam, T sigma, const McSide<T>& o, T& jn, T& fd, T& ftau, T& fs1, T& fs2,
-                                       T& fs3) {
+template <int DIR, typename T> __device__ inline void mcl_side_fluxes(T gam, T sigma, Side<T>& o) {
   const T e2b2 = ((((sq(o.ex) + sq(o.ey)) + sq(o.ez)) + sq(o.bx)) + sq(o.by)) + sq(o.bz);
   const T w = T(1) / sqrt(((T(1) - sq(o.vx)) - sq(o.vy)) - sq(o.vz));
   const T edv = (o.ex * o.vx + o.ey * o.vy) + o.ez * o.vz;
@@ -197,132 +174,125 @@ __device__ inline void mcl_side_fluxes(T gam, T sigma, const McSide<T>& o, T& jn
   const T h = o.rho * (T(1) + eps) + o.p;
   const T hw2 = h * sq(w);
   if constexpr (DIR == 0) {
-    jn = (sigma * w) * ((o.ex + (o.bz * o.vy - o.by * o.vz)) - edv * o.vx) + o.q * o.vx;
-    fd = o.d * o.vx;
-    ftau = (o.bz * o.ey - o.by * o.ez) + hw2 * o.vx;
-    fs1 = ((((-sq(o.ex)) - sq(o.bx)) + hw2 * sq(o.vx)) + T(0.5) * e2b2) + o.p;
-    fs2 = ((-(o.ex * o.ey)) - o.bx * o.by) + (hw2 * o.vx) * o.vy;
-    fs3 = ((-(o.ex * o.ez)) - o.bx * o.bz) + (hw2 * o.vx) * o.vz;
+    o.jn = (sigma * w) * ((o.ex + (o.bz * o.vy - o.by * o.vz)) - edv * o.vx) + o.q * o.vx;
+    o.fd = o.d * o.vx;
+    o.ftau = (o.bz * o.ey - o.by * o.ez) + hw2 * o.vx;
+    o.fs1 = ((((-sq(o.ex)) - sq(o.bx)) + hw2 * sq(o.vx)) + T(0.5) * e2b2) + o.p;
+    o.fs2 = ((-(o.ex * o.ey)) - o.bx * o.by) + (hw2 * o.vx) * o.vy;
+    o.fs3 = ((-(o.ex * o.ez)) - o.bx * o.bz) + (hw2 * o.vx) * o.vz;
   } else {
-    jn = (sigma * w) * ((o.ey + (o.bx * o.vz - o.bz * o.vx)) - edv * o.vy) + o.q * o.vy;
-    fd = o.d * o.vy;
-    ftau = (o.bx * o.ez - o.bz * o.ex) + hw2 * o.vy;
-    fs1 = ((-(o.ex * o.ey)) - o.bx * o.by) + (hw2 * o.vx) * o.vy;
-    fs2 = ((((-sq(o.ey)) - sq(o.by)) + hw2 * sq(o.vy)) + T(0.5) * e2b2) + o.p;
-    fs3 = ((-(o.ey * o.ez)) - o.by * o.bz) + (hw2 * o.vy) * o.vz;
+    o.jn = (sigma * w) * ((o.ey + (o.bx * o.vz - o.bz * o.vx)) - edv * o.vy) + o.q * o.vy;
+    o.fd = o.d * o.vy;
+    o.ftau = (o.bx * o.ez - o.bz * o.ex) + hw2 * o.vy;
+    o.fs1 = ((-(o.ex * o.ey)) - o.bx * o.by) + (hw2 * o.vx) * o.vy;
+    o.fs2 = ((((-sq(o.ey)) - sq(o.by)) + hw2 * sq(o.vy)) + T(0.5) * e2b2) + o.p;
+    o.fs3 = ((-(o.ey * o.ez)) - o.by * o.bz) + (hw2 * o.vy) * o.vz;
   }
+}
+
+// One quantity's left and right face values between a cell and its +x (DIR 0)
+// or +y (DIR 1) neighbour (u_L = u_i + FAC mcl(.), u_R = u_{i+1} - FAC mcl(.),
+// FAC = 0.5), and of the tangential E and B pair the "_m" states: the cell
+// value negated, the slope kept (16_hll_flow_mcl.f95:634-655, 708-737)
+template <int F, int DIR, int KIND, typename ST, typename T>
+__device__ inline void mcl_take(int slop, const Sten<4, ST>& s, Side<T>& L, Side<T>& R) {
+  const T um = (T)s.v[0], u0 = (T)s.v[1], u1 = (T)s.v[2], u2 = (T)s.v[3];
+  const T sl = T(0.5) * mcl_slope(u1 - u0, u0 - um, KIND ? KIND : slop);
+  const T sr = T(0.5) * mcl_slope(u2 - u1, u1 - u0, KIND ? KIND : slop);
+  face_slot<F>(L) = u0 + sl;
+  face_slot<F>(R) = u1 - sr;
+  if constexpr (F == (DIR == 0 ? F_EZ : F_EX)) {
+    L.em = (-u0) + sl;
+    R.em = (-u1) - sr;
+  }
+  if constexpr (F == (DIR == 0 ? F_BY : F_BZ)) {
+    L.bm = (-u0) + sl;
+    R.bm = (-u1) - sr;
+  }
+}
+
+// The states of one face from the MC limiter with their physical fluxes
+// (16_hllc_flow_mcl.f95:1760-2479 forms the same ones).  A quantity's four
+// values are loaded MCL_AHEAD quantities before it is reconstructed, and its
+// two states are pinned where they are formed: left to itself the compiler put
+// the reconstruction where the states are used, which held all nineteen
+// stencils in registers (63-168 VGPRs spilled in FP64; none now) and exposed
+// the loads.  HLL + MC FP64 step at 2048x4096 / 300x700: 7.1 ms / 188 us
+// before; 2 ahead 3.66 / 102.6, 4 ahead 3.47 / 102.1, 6 ahead 3.50 / 102.5.
+constexpr int MCL_AHEAD = 4;
+template <int DIR, int KIND, bool STAGE_KIN, typename ST, typename T, int... Q>
+__device__ inline void mcl_fields(const Planes& P, int slop, const Cell& c, Side<T>& L, Side<T>& R,
+                                  std::integer_sequence<int, Q...>) {
+  constexpr int N = sizeof...(Q), AH = MCL_AHEAD;
+  Sten<4, ST> b[AH + 1];
+  auto pre = [&](auto t) {
+    if constexpr (t() < AH) face_load<t(), DIR, STAGE_KIN>(P, c, b[t()]);
+  };
+  auto one = [&](auto t) {
+    if constexpr (t() + AH < N) face_load<t() + AH, DIR, STAGE_KIN>(P, c, b[(t() + AH) % (AH + 1)]);
+    mcl_take<t(), DIR, KIND>(slop, b[t() % (AH + 1)], L, R);
+    asm volatile("" : "+v"(face_slot<t()>(L)), "+v"(face_slot<t()>(R)));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  (pre(std::integral_constant<int, Q>()), ...);
+  (one(std::integral_constant<int, Q>()), ...);
+}
+template <int F, int DIR, bool STAGE_KIN, typename ST, typename T>
+__device__ inline void mcl_one(const Planes& P, int slop, const Cell& c, Side<T>& L, Side<T>& R) {
+  Sten<4, ST> s;
+  face_load<F, DIR, STAGE_KIN>(P, c, s);
+  mcl_take<F, DIR, 0>(slop, s, L, R);
+}
+template <int DIR, bool STAGE_KIN, typename ST, typename T>
+__device__ inline void mcl_sides(const Planes& P, const Scheme& S, const Cell& c, Side<T>& L, Side<T>& R) {
+  // the default slope has its own body: chosen per quantity, the compiler
+  // evaluated all three slopes and selected
+  if (S.slop == 2) mcl_fields<DIR, 2, STAGE_KIN, ST>(P, S.slop, c, L, R, std::make_integer_sequence<int, F_JN>());
+  else mcl_fields<DIR, 0, STAGE_KIN, ST>(P, S.slop, c, L, R, std::make_integer_sequence<int, F_JN>());
+  mcl_side_fluxes<DIR>((T)S.gamma, (T)S.sigma, L);
+  mcl_side_fluxes<DIR>((T)S.gamma, (T)S.sigma, R);
 }
 
 // 0.5 (A_L + A_R - Sp (U_R - U_L)) with Sp = 1 (16_hll_flow_mcl.f95:1259-1396)
 template <typename T> __device__ inline T mcl_lf(T al, T ar, T ul, T ur) { return T(0.5) * ((al + ar) - (ur - ul)); }
 
-// the fluxes of the face between the cells at c and c+st, DIR 0 = x (FX_*
-// slots), 1 = y (FY_* slots)
-template <int DIR, typename ST, typename T>
+// the fluxes of the face between the cell at c and its +x (DIR 0, FX_* slots)
+// or +y neighbour (DIR 1, FY_*)
+template <int DIR, bool STAGE_KIN, typename ST, typename T>
 __device__ inline void mcl_face(const Planes& P, const Scheme& S, const Cell& c, T* f) {
-  McSide<T> L, R;
-  T e0[2], es[2], b0[2], bs[2];  // cell values and half-slopes of the "_m" pair
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_PSI), c, L.psi, R.psi);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_PHI), c, L.phi, R.phi);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_EX), c, L.ex, R.ex, DIR == 1 ? e0 : (T*)nullptr, DIR == 1 ? es : (T*)nullptr);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_EY), c, L.ey, R.ey);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_EZ), c, L.ez, R.ez, DIR == 0 ? e0 : (T*)nullptr, DIR == 0 ? es : (T*)nullptr);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_BX), c, L.bx, R.bx);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_BY), c, L.by, R.by, DIR == 0 ? b0 : (T*)nullptr, DIR == 0 ? bs : (T*)nullptr);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_BZ), c, L.bz, R.bz, DIR == 1 ? b0 : (T*)nullptr, DIR == 1 ? bs : (T*)nullptr);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_Q), c, L.q, R.q);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_D), c, L.d, R.d);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_TAU), c, L.tau, R.tau);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_SX), c, L.sx, R.sx);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_SY), c, L.sy, R.sy);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_SZ), c, L.sz, R.sz);
-  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_VX), c, L.vx, R.vx);
-  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_VY), c, L.vy, R.vy);
-  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_VZ), c, L.vz, R.vz);
-  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_P), c, L.p, R.p);
-  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_RHO), c, L.rho, R.rho);
-  // "_m" states: the cell value negated, the slope kept
-  // (16_hll_flow_mcl.f95:634-655, 708-737)
-  const T em_l = (-e0[0]) + es[0], em_r = (-e0[1]) - es[1];
-  const T bm_l = (-b0[0]) + bs[0], bm_r = (-b0[1]) - bs[1];
-  T jl, fdl, ftl, f1l, f2l, f3l, jr, fdr, ftr, f1r, f2r, f3r;
-  mcl_side_fluxes<DIR>((T)S.gamma, (T)S.sigma, L, jl, fdl, ftl, f1l, f2l, f3l);
-  mcl_side_fluxes<DIR>((T)S.gamma, (T)S.sigma, R, jr, fdr, ftr, f1r, f2r, f3r);
+  Side<T> L, R;
+  mcl_sides<DIR, STAGE_KIN, ST>(P, S, c, L, R);
   if constexpr (DIR == 0) {
     f[FX_EXPSI] = mcl_lf(L.ex, R.ex, L.psi, R.psi);
     f[FX_BXPHI] = mcl_lf(L.bx, R.bx, L.phi, R.phi);
     f[FX_PHIBX] = mcl_lf(L.phi, R.phi, L.bx, R.bx);
-    f[FX_EZBY] = -mcl_lf(em_l, em_r, L.by, R.by);
+    f[FX_EZBY] = -mcl_lf(L.em, R.em, L.by, R.by);
     f[FX_EYBZ] = mcl_lf(L.ey, R.ey, L.bz, R.bz);
     f[FX_PSIEX] = mcl_lf(L.psi, R.psi, L.ex, R.ex);
     f[FX_BZEY] = mcl_lf(L.bz, R.bz, L.ey, R.ey);
-    f[FX_BYEZ] = -mcl_lf(bm_l, bm_r, L.ez, R.ez);
-    f[FX_J] = mcl_lf(jl, jr, L.q, R.q);
-    f[FX_FD] = mcl_lf(fdl, fdr, L.d, R.d);
-    f[FX_FTAU] = mcl_lf(ftl, ftr, L.tau, R.tau);
-    f[FX_FSX] = mcl_lf(f1l, f1r, L.sx, R.sx);
-    f[FX_FSY] = mcl_lf(f2l, f2r, L.sy, R.sy);
-    f[FX_FSZ] = mcl_lf(f3l, f3r, L.sz, R.sz);
+    f[FX_BYEZ] = -mcl_lf(L.bm, R.bm, L.ez, R.ez);
+    f[FX_J] = mcl_lf(L.jn, R.jn, L.q, R.q);
+    f[FX_FD] = mcl_lf(L.fd, R.fd, L.d, R.d);
+    f[FX_FTAU] = mcl_lf(L.ftau, R.ftau, L.tau, R.tau);
+    f[FX_FSX] = mcl_lf(L.fs1, R.fs1, L.sx, R.sx);
+    f[FX_FSY] = mcl_lf(L.fs2, R.fs2, L.sy, R.sy);
+    f[FX_FSZ] = mcl_lf(L.fs3, R.fs3, L.sz, R.sz);
   } else {
     f[FY_EYPSI] = mcl_lf(L.ey, R.ey, L.psi, R.psi);
     f[FY_BYPHI] = mcl_lf(L.by, R.by, L.phi, R.phi);
     f[FY_EZBX] = mcl_lf(L.ez, R.ez, L.bx, R.bx);
     f[FY_PHIBY] = mcl_lf(L.phi, R.phi, L.by, R.by);
-    f[FY_EXBZ] = -mcl_lf(em_l, em_r, L.bz, R.bz);
-    f[FY_BZEX] = -mcl_lf(bm_l, bm_r, L.ex, R.ex);
+    f[FY_EXBZ] = -mcl_lf(L.em, R.em, L.bz, R.bz);
+    f[FY_BZEX] = -mcl_lf(L.bm, R.bm, L.ex, R.ex);
     f[FY_PSIEY] = mcl_lf(L.psi, R.psi, L.ey, R.ey);
     f[FY_BXEZ] = mcl_lf(L.bx, R.bx, L.ez, R.ez);
-    f[FY_J] = mcl_lf(jl, jr, L.q, R.q);
-    f[FY_FD] = mcl_lf(fdl, fdr, L.d, R.d);
-    f[FY_FTAU] = mcl_lf(ftl, ftr, L.tau, R.tau);
-    f[FY_FSX] = mcl_lf(f1l, f1r, L.sx, R.sx);
-    f[FY_FSY] = mcl_lf(f2l, f2r, L.sy, R.sy);
-    f[FY_FSZ] = mcl_lf(f3l, f3r, L.sz, R.sz);
+    f[FY_J] = mcl_lf(L.jn, R.jn, L.q, R.q);
+    f[FY_FD] = mcl_lf(L.fd, R.fd, L.d, R.d);
+    f[FY_FTAU] = mcl_lf(L.ftau, R.ftau, L.tau, R.tau);
+    f[FY_FSX] = mcl_lf(L.fs1, R.fs1, L.sx, R.sx);
+    f[FY_FSY] = mcl_lf(L.fs2, R.fs2, L.sy, R.sy);
+    f[FY_FSZ] = mcl_lf(L.fs3, R.fs3, L.sz, R.sz);
   }
-}
-
-// The face states of HLLC with the MC limiter (flux_solver = 4,
-// 16_hllc_flow_mcl.f95:1760-2479, the states and fluxes of hll_flow), as
-// the HLLC solve reads them
-template <int DIR, typename ST, typename T>
-__device__ inline void mcl_sides(const Planes& P, const Scheme& S, const Cell& c, Side<T>& L, Side<T>& R) {
-  McSide<T> l, r;
-  T e0[2], es[2], b0[2], bs[2];
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_PSI), c, l.psi, r.psi);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_PHI), c, l.phi, r.phi);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_EX), c, l.ex, r.ex, DIR == 1 ? e0 : (T*)nullptr, DIR == 1 ? es : (T*)nullptr);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_EY), c, l.ey, r.ey);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_EZ), c, l.ez, r.ez, DIR == 0 ? e0 : (T*)nullptr, DIR == 0 ? es : (T*)nullptr);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_BX), c, l.bx, r.bx);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_BY), c, l.by, r.by, DIR == 0 ? b0 : (T*)nullptr, DIR == 0 ? bs : (T*)nullptr);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_BZ), c, l.bz, r.bz, DIR == 1 ? b0 : (T*)nullptr, DIR == 1 ? bs : (T*)nullptr);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_Q), c, l.q, r.q);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_D), c, l.d, r.d);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_TAU), c, l.tau, r.tau);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_SX), c, l.sx, r.sx);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_SY), c, l.sy, r.sy);
-  mcl_rec<DIR>(S.slop, stage_src<ST>(P, S_SZ), c, l.sz, r.sz);
-  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_VX), c, l.vx, r.vx);
-  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_VY), c, l.vy, r.vy);
-  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_VZ), c, l.vz, r.vz);
-  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_P), c, l.p, r.p);
-  mcl_rec<DIR>(S.slop, kin_src<ST>(P, K_RHO), c, l.rho, r.rho);
-  Side<T>* sd[2] = {&L, &R};
-  const McSide<T>* ms[2] = {&l, &r};
-#pragma unroll
-  for (int t = 0; t < 2; t++) {
-    Side<T>& o = *sd[t];
-    const McSide<T>& m = *ms[t];
-    o.psi = m.psi; o.phi = m.phi; o.ex = m.ex; o.ey = m.ey; o.ez = m.ez;
-    o.bx = m.bx; o.by = m.by; o.bz = m.bz; o.q = m.q; o.d = m.d; o.tau = m.tau;
-    o.sx = m.sx; o.sy = m.sy; o.sz = m.sz; o.vx = m.vx; o.vy = m.vy; o.vz = m.vz; o.p = m.p; o.rho = m.rho;
-    mcl_side_fluxes<DIR>((T)S.gamma, (T)S.sigma, m, o.jn, o.fd, o.ftau, o.fs1, o.fs2, o.fs3);
-  }
-  // "_m" states: the cell value negated, the slope kept
-  L.em = (-e0[0]) + es[0];
-  R.em = (-e0[1]) - es[1];
-  L.bm = (-b0[0]) + bs[0];
-  R.bm = (-b0[1]) - bs[1];
 }
 
 // ---------------------------------------------------------------------------
@@ -454,15 +424,18 @@ __device__ __forceinline__ void face_pair(const Geom& g, const Planes& P, const 
     T xseed = T(0), vlast = T(0);
     Side<T> sl, sr;
     if (seed) {
-      mcl_sides<1, ST>(P, S, cc, sl, sr);
+      mcl_one<F_EX, 1, STAGE_KIN, ST>(P, S.slop, cc, sl, sr);
+      mcl_one<F_EZ, 1, STAGE_KIN, ST>(P, S.slop, cc, sl, sr);
+      mcl_one<F_BX, 1, STAGE_KIN, ST>(P, S.slop, cc, sl, sr);
+      mcl_one<F_BZ, 1, STAGE_KIN, ST>(P, S.slop, cc, sl, sr);
       xseed = hlle_y_ery<T, true>(sl, sr);
     }
-    mcl_sides<0, ST>(P, S, cc, sl, sr);
+    mcl_sides<0, STAGE_KIN, ST>(P, S, cc, sl, sr);
     int code = SOLVER == 3 ? hlle_mcl_face<0>((T)S.gamma, sl, sr, f, seed, xseed, vlast)
                            : hllc_x<T, true>(sl, sr, f, seed, xseed, &vlast);
     if (code) report(st, code, i, j);
     put_x(f);
-    mcl_sides<1, ST>(P, S, cc, sl, sr);
+    mcl_sides<1, STAGE_KIN, ST>(P, S, cc, sl, sr);
     T unused;
     code = SOLVER == 3 ? hlle_mcl_face<1>((T)S.gamma, sl, sr, f, seed, vlast, unused)
                        : hllc_y<T, true>(sl, sr, f, seed, vlast);
@@ -475,7 +448,7 @@ __device__ __forceinline__ void face_pair(const Geom& g, const Planes& P, const 
     auto face = [&](auto dir) {
       constexpr int D = decltype(dir)::value;
       if constexpr (SOLVER == 1) lax_face<D, ST>(g, P, S, i, j, f);
-      else mcl_face<D, ST>(P, S, cc, f);
+      else mcl_face<D, STAGE_KIN, ST>(P, S, cc, f);
       if constexpr (D == 0) put_x(f);
       else put_y(f);
     };
@@ -569,15 +542,13 @@ __device__ __forceinline__ void face_pair(const Geom& g, const Planes& P, const 
   }
 }
 
-// Waves per SIMD k_faces is built for (a register bound).  Unbounded, the
-// MCL solvers' face pairs need 177-181 VGPRs in FP32 (2 waves per SIMD) and
-// past 256 in FP64 (1 wave): bounded to 3 (FP32, 14-16 VGPRs spilled) the
-// face pass measured 18-19 % faster at 2048x4096, and to 2 (FP64) HLL-MCL
-// 8 % and HLLC-MCL 5 % faster, HLLE-MCL (176 spilled) 3 % slower, so it
-// stays unbounded.  The other solvers fit their waves unbounded.
+// Waves per SIMD k_faces is built for (a register bound).  The MCL solvers
+// need 197 VGPRs in FP64 and 125-143 in FP32 and the bound keeps the compiler
+// from taking more than their waves leave; the other solvers fit their waves
+// unbounded.
 template <typename T, int SOLVER>
 constexpr int faces_min_waves() {
-  if constexpr (sizeof(T) == 8) return SOLVER == 2 || SOLVER == 4 ? 2 : 1;
+  if constexpr (sizeof(T) == 8) return SOLVER >= 2 && SOLVER <= 4 ? 2 : 1;
   else return SOLVER >= 2 && SOLVER <= 4 ? 3 : 1;
 }
 
@@ -661,10 +632,11 @@ static_assert(offsetof(MarchArgs, P) == 0, "argument block layout");
 
 // Waves per SIMD the marching kernel is built for, a register bound (the
 // compiler spills past it).  Measured per step at 2048x4096:
-//   FP64: 2 for every solver.  HLLC fits 237 VGPRs; the others need a few
-//     more than 256 and ran 1 wave per SIMD unbounded: bounded, HLL spills
-//     2-12 VGPRs and runs 36 % faster, HLLE (one y-row buffer, below) 36 %,
-//     Lax-Friedrichs 32 %, the MCL solvers (63-114 spilled) 17-20 %;
+//   FP64: 2 for every solver.  HLLC fits 227 VGPRs, the MCL solvers 184-229;
+//     the others need a few more than 256 and ran 1 wave per SIMD unbounded:
+//     bounded, HLL runs 36 % faster, HLLE (one y-row buffer, below) 36 %,
+//     Lax-Friedrichs 32 %.  3 waves (168 VGPRs) spill 22-40 under HLLC and
+//     ran 12 % slower;
 //   FP32: 3.  With the stencils loaded ahead, 4 waves (128 VGPRs) spill
 //     and ran 3-6 % slower under HLLC, HLLE and HLL, 19 % under HLL + MC.
 template <typename T, int SOLVER>
