@@ -129,9 +129,18 @@ __global__ void k_startconvar(Geom g, Planes P, Scheme S) {
   P.c[C_SX][k] = c.sx; P.c[C_SY][k] = c.sy; P.c[C_SZ][k] = c.sz; P.c[C_W][k] = c.w;
 }
 
-// cleanvarint, 07_clean_var.f95:18-60
-__global__ void k_cleanvarint(Geom g, Planes P) {
+// cleanvarint, 07_clean_var.f95:18-60, and the step's counters and fix-up
+// records (main_cueva_code.f95:189-193): a fill of their own was one launch
+// more of some 6 us from the host
+__global__ void k_cleanvarint(Geom g, Planes P, DevStatus* st) {
   INTERIOR_IJ
+  if (i == 0 && j == 0) {
+    for (int d = 0; d < 3; d++) {
+      st->cnt[d] = 0;
+      st->nrec[d] = 0;
+    }
+    st->fallback = 0;
+  }
   for (int a = 0; a < A_N; a++) { P.ints[a][k] = 0.0; P.fins[a][k] = 0.0; }
 }
 
