@@ -654,10 +654,10 @@ constexpr int march_y_buffers() {
   return SOLVER == 6 ? 1 : 2;
 }
 
-// Wavefronts per block = face rows per tile step.  4 everywhere by default;
-// FP32 HLL/HLLC may take 8 (a tile step then re-reads 5 halo rows per 8 face
-// rows instead of per 4; two 61 KB blocks per CU still give 4 waves per SIMD)
-// but measured the same step time at 2048x4096, so the smaller block stays.
+// Wavefronts per block = face rows per tile step: 4.  More re-read fewer halo
+// rows (a tile step reads MW + 5), but the barriers then wait for more of
+// them: HLLC + MP5 at 2048x4096 with 4 / 6 / 8 waves, FP64 5.12 / 6.45 / 5.49
+// ms per step, FP32 4.15 / 4.93 / 4.53 (12 waves 4.30).
 #ifndef CUEVA_MARCH_F32_BLOCK_WAVES
 #define CUEVA_MARCH_F32_BLOCK_WAVES 4
 #endif
@@ -689,9 +689,9 @@ k_faces_march(MarchArgs args) {
     // The arguments (plane pointers, geometry, scheme constants) are read
     // again from the kernel's argument block every tile step rather than
     // held in scalar registers across the loop, where they do not fit and
-    // spill into vector-register lanes (FP64 HLLC: 156 SGPRs spilled, none
-    // this way; FP32 HLLC: 147 VGPRs against 139).  FP64 HLL keeps them:
-    // re-reading measured 24 % slower there.
+    // spill into vector-register lanes: kept, the FP32 forms measured 8 %
+    // slower at 2048x4096, FP64 HLLC the same.  FP64 HLL keeps them:
+    // re-reading measured 16 % slower there.
     constexpr bool REREAD = sizeof(T) == 4 || SOLVER != 5;
     const __attribute__((address_space(4))) MarchArgs* ap =
         (const __attribute__((address_space(4))) MarchArgs*)__builtin_amdgcn_kernarg_segment_ptr();
