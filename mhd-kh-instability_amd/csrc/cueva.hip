@@ -550,7 +550,12 @@ static void io_work(IoJob& j, PinnedPair& p) {
   }
   finish(k);
   finish(k ^ 1);
-  if (!ok) j.err.store(1, std::memory_order_relaxed);
+  if (!ok) {
+    // a kernel that was launched without its event being recorded, or whose
+    // event could not be waited for, still reads or writes a buffer
+    (void)hipStreamSynchronize(j.c->stream);
+    j.err.store(1, std::memory_order_relaxed);
+  }
 }
 
 // row by row with strided copies: device pointers given in place of host
