@@ -17,9 +17,11 @@
  *    is in the restart order psi phi Bx By Bz Vx Vy Vz Ex Ey Ez q rho p
  *    (22_writer.f95:1116-1172).
  *  - Calls on one ctx are ordered on the ctx's HIP stream; only
- *    cueva_step, cueva_c2p, cueva_download*, the counter, record and error
- *    queries, cueva_reduce_globals and cueva_sync wait for the device.  A
- *    ctx is not thread safe.
+ *    cueva_step, cueva_c2p, cueva_upload*, cueva_download*, the counter,
+ *    record and error queries, cueva_plane_range, cueva_reduce_globals,
+ *    cueva_max_speed, the timing calls, cueva_set_c2p_params and cueva_sync
+ *    wait for the device: an array given to them is the caller's again on
+ *    return.  A ctx is not thread safe.
  *  - Failures: where the reference prints and stops, the device records the
  *    first failure in the reference's own order (the launch that failed
  *    first; in it, the first cell of the reference's loop, j outer, i inner)

@@ -559,19 +559,22 @@ static void io_work(IoJob& j, PinnedPair& p) {
 }
 
 // row by row with strided copies: device pointers given in place of host
-// arrays, and where no pinned memory is to be had
+// arrays, and where no pinned memory is to be had.  The stream is waited for,
+// also after a copy that could not be queued: the caller's array is then free.
 static int copy_planes_strided(cueva_ctx* c, double* const* planes, int n, double* host, bool up) {
   const Geom& g = c->g;
   const size_t hw = (size_t)(g.imax + 13), hh = (size_t)(g.jmax + 13), row = hw * sizeof(double);
-  for (int k = 0; k < n; k++) {
+  hipError_t e = hipSuccess;
+  for (int k = 0; k < n && e == hipSuccess; k++) {
     double* h = host + (size_t)k * hw * hh;
     const size_t pitch = (size_t)g.pitch * sizeof(double);
     if (up)
-      HIPCHK(hipMemcpy2DAsync(planes[k] + (X0 - GH), pitch, h, row, row, hh, hipMemcpyHostToDevice, c->stream));
+      e = hipMemcpy2DAsync(planes[k] + (X0 - GH), pitch, h, row, row, hh, hipMemcpyHostToDevice, c->stream);
     else
-      HIPCHK(hipMemcpy2DAsync(h, row, planes[k] + (X0 - GH), pitch, row, hh, hipMemcpyDeviceToHost, c->stream));
+      e = hipMemcpy2DAsync(h, row, planes[k] + (X0 - GH), pitch, row, hh, hipMemcpyDeviceToHost, c->stream);
   }
-  return CUEVA_OK;
+  const hipError_t w = hipStreamSynchronize(c->stream);
+  return e == hipSuccess && w == hipSuccess ? CUEVA_OK : CUEVA_E_HIP;
 }
 
 // n planes (at most 32) up from or down to a host array; the caller's array is

@@ -78,3 +78,33 @@ fail("hipEventRecord", %d)
 assert L.cueva_download(s.ctx, ptr(prims), None) == 2
 assert rt.fake_pending() == 0
 """ % (after, after), ni, nj)
+
+
+@pytest.mark.parametrize("ni,nj", GRIDS)
+def test_strided_copies_are_over_on_return(standin, ni, nj):
+    """Device memory given in place of a host array, and no pinned memory to be had: the caller's
+    array is its own again when the call returns."""
+    run(standin, """
+dev = ctypes.c_void_p()
+assert rt.hipMalloc(ctypes.byref(dev), prims.nbytes) == 0
+mem = np.ctypeslib.as_array(ctypes.cast(dev, P), shape=prims.shape)
+mem[:] = prims
+assert L.cueva_upload_prims(s.ctx, ctypes.cast(dev, P)) == 0
+mem[:] = -1.0
+assert np.array_equal(s.download(cons=False), prims)
+mem[:5] = cons
+assert L.cueva_upload_cons(s.ctx, ctypes.cast(dev, P)) == 0 and rt.fake_pending() == 0
+mem[:] = -1.0
+assert L.cueva_download(s.ctx, ctypes.cast(dev, P), None) == 0 and rt.fake_pending() == 0
+assert np.array_equal(mem, prims) and np.array_equal(s.download()[1], cons)
+""", ni, nj)
+    run(standin, """
+fail("hipHostMalloc", 0, 1000000)
+a = cons.copy()
+assert L.cueva_upload_cons(s.ctx, ptr(a)) == 0 and rt.fake_pending() == 0
+a[:] = -1.0
+assert np.array_equal(s.download()[1], cons)
+# a copy that cannot be queued: the ones before it are over too
+fail("hipMemcpy2DAsync", 2)
+assert L.cueva_upload_cons(s.ctx, ptr(a)) == 2 and rt.fake_pending() == 0
+""", ni, nj)
