@@ -59,6 +59,7 @@ struct PinnedPair {
 
 struct cueva_ctx {
   cueva_params prm;
+  int dev;  // the device that was current at creation
   Geom g;
   Scheme S;
   Planes P;
@@ -323,7 +324,10 @@ extern "C" int cueva_create(const cueva_params* p, cueva_ctx** out) {
   const int nstage = p->rec_prim ? S.lmax * 7 : 0;  // stage primitives of REC_PRIM = 1
   const int nplanes = P_N + C_N + 2 * S_N + FX_N + FY_N + MAXL * R_N + 2 * A_N + nstage;
   c->bytes = (int64_t)nplanes * g.plane * (int64_t)sizeof(double);
-  if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) { delete c; return CUEVA_E_HIP; }
+  if (hipGetDevice(&c->dev) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
+    delete c;
+    return CUEVA_E_HIP;
+  }
   if (hipMalloc(&c->base, (size_t)c->bytes) != hipSuccess) {
     hipStreamDestroy(c->stream);
     delete c;
@@ -511,7 +515,7 @@ struct IoJob {
   cueva_ctx* c;
   PlaneList pl;
   double* host;
-  int up, w, hh, run, runs, dev;
+  int up, w, hh, run, runs;
   std::atomic<int> next;
   std::atomic<int> err;
 };
@@ -577,6 +581,22 @@ static int copy_planes_strided(cueva_ctx* c, double* const* planes, int n, doubl
   return e == hipSuccess && w == hipSuccess ? CUEVA_OK : CUEVA_E_HIP;
 }
 
+// The context's device made current while this lives: a copy may be queued on
+// any device's stream, but not a kernel or an event, and a thread other than
+// the creating one (a writer's) may have another device current.
+struct CurrentDevice {
+  int was = 0;
+  bool ok, moved = false;
+  explicit CurrentDevice(int dev) {
+    ok = hipGetDevice(&was) == hipSuccess;
+    if (ok && was != dev) ok = moved = hipSetDevice(dev) == hipSuccess;
+  }
+  ~CurrentDevice() {
+    if (moved) (void)hipSetDevice(was);
+  }
+  CurrentDevice(const CurrentDevice&) = delete;
+};
+
 // n planes (at most 32) up from or down to a host array; the caller's array is
 // read or written in full when this returns
 static int copy_planes(cueva_ctx* c, double* const* planes, int n, double* host, bool up) {
@@ -602,7 +622,8 @@ static int copy_planes(cueva_ctx* c, double* const* planes, int n, double* host,
   j.runs = (int)((total + run - 1) / run);
   j.next = 0;
   j.err = 0;
-  if (hipGetDevice(&j.dev) != hipSuccess) return CUEVA_E_HIP;
+  const CurrentDevice on(c->dev);
+  if (!on.ok) return CUEVA_E_HIP;
   int threads = 1;
   if (bytes > 4 * IO_CHUNK) {
     cpu_set_t set;
@@ -619,7 +640,7 @@ static int copy_planes(cueva_ctx* c, double* const* planes, int n, double* host,
   for (int t = 1; t < threads; t++) {
     try {
       th[t] = std::thread([&j, c, t]() {
-        if (hipSetDevice(j.dev) == hipSuccess) io_work(j, c->io[t]);
+        if (hipSetDevice(c->dev) == hipSuccess) io_work(j, c->io[t]);
       });
     } catch (const std::exception&) {  // no more threads: the others take its runs
       break;

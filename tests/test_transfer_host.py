@@ -108,3 +108,22 @@ assert np.array_equal(s.download()[1], cons)
 fail("hipMemcpy2DAsync", 2)
 assert L.cueva_upload_cons(s.ctx, ptr(a)) == 2 and rt.fake_pending() == 0
 """, ni, nj)
+
+
+@pytest.mark.parametrize("ni,nj", GRIDS)
+def test_transfers_with_another_device_current(standin, ni, nj):
+    """A copy to or from a context is taken from a thread whose current device is another one, which stays current."""
+    run(standin, """
+rt.hipSetDevice(3)
+d = ctypes.c_int()
+with cueva.Solver(p) as t:
+    assert L.cueva_upload_prims(t.ctx, ptr(prims)) == 0
+    rt.hipSetDevice(0)
+    assert L.cueva_upload_cons(t.ctx, ptr(cons)) == 0
+    a, b = t.download()
+    assert np.array_equal(a, prims) and np.array_equal(b, cons) and np.array_equal(t.plane(0, 3), prims[3])
+    assert rt.hipGetDevice(ctypes.byref(d)) == 0 and d.value == 0
+    rt.hipSetDevice(3)
+    assert L.cueva_upload_cons(t.ctx, ptr(-cons)) == 0
+    assert np.array_equal(t.download()[1], -cons)
+""", ni, nj)
