@@ -493,14 +493,14 @@ static bool io_reserve(PinnedPair& p, size_t bytes) {
   io_release(p);
   for (int k = 0; k < 2; k++) {
     void* b = nullptr;
-    if (hipHostMalloc(&b, bytes, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess) {
-      (void)hipGetLastError();
-      io_release(p);
-      return false;
+    bool ok = hipHostMalloc(&b, bytes, hipHostMallocCoherent | hipHostMallocMapped) == hipSuccess;
+    if (ok) {
+      p.buf[k] = (double*)b;
+      ok = hipEventCreateWithFlags(&p.done[k], hipEventDisableTiming) == hipSuccess;
+      if (!ok) p.done[k] = nullptr;
     }
-    p.buf[k] = (double*)b;
-    if (hipEventCreateWithFlags(&p.done[k], hipEventDisableTiming) != hipSuccess) {
-      p.done[k] = nullptr;
+    if (!ok) {
+      (void)hipGetLastError();  // the transfer goes on without: no later call reports this
       io_release(p);
       return false;
     }

@@ -127,3 +127,19 @@ with cueva.Solver(p) as t:
     assert L.cueva_upload_cons(t.ctx, ptr(-cons)) == 0
     assert np.array_equal(t.download()[1], -cons)
 """, ni, nj)
+
+
+@pytest.mark.parametrize("after", [0, 1, 3])
+@pytest.mark.parametrize("call", ["hipHostMalloc", "hipEventCreateWithFlags"])
+def test_transfers_without_pinned_buffers(standin, call, after):
+    """Where a buffer or its event cannot be had, for any of the threads, the transfer is done without it
+    and the refusal is not reported by a later call."""
+    run(standin, """
+fail(%r, %d, 1000000)
+assert L.cueva_upload_prims(s.ctx, ptr(prims)) == 0
+assert np.array_equal(s.download(cons=False), prims)
+assert rt.hipGetLastError() == 0
+fail(%r, 0, 0)
+assert L.cueva_upload_prims(s.ctx, ptr(-prims)) == 0
+assert np.array_equal(s.download(cons=False), -prims)
+""" % (call, after, call), 400, 800)
