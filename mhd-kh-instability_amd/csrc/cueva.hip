@@ -1128,10 +1128,13 @@ static void swap_stage(cueva_ctx* c) {
   }
 }
 
-// Whether the state of stage l of step h out of nsteps (0-based) stays after
-// the call: it is then kept in full (store_stage).
+// Whether the state of stage l of step h out of nsteps (0-based) is kept in
+// full (store_stage): the one that stays after the call, and with MIRK2 and one
+// stage every one, because the closing electric field reads that stage's B
+// (mirk_final_e; times a velocity of zero, which NaN left by an earlier state
+// survives).
 static int stays(const cueva_ctx* c, int l, int h, int nsteps) {
-  return !c->march || (l == c->S.lmax - 1 && h == nsteps - 1);
+  return !c->march || (l == c->S.lmax - 1 && (h == nsteps - 1 || (l == 0 && c->prm.mirk == 2)));
 }
 
 // U^{n+1}, left by the last marching launch in rhs[L][0..13], becomes the
