@@ -278,14 +278,24 @@ template <int ORD, typename T> __device__ inline void mp_face(const T* v, T& L, 
 
 // Same with the positivity fallback of mp5.f95:177-216 (p and rho slots): at
 // each cell, first "up < 0" then "um < 0" rewrites both interface values.
-// Where every stencil value is positive and within a factor 1.9 of the
+// Where every stencil value is positive and within a factor CALM of the
 // others, no interface value of either cell can be negative, whatever the
-// limiter does: the unlimited ones are at least (76 - 16 * 1.9) / 60 (MP5;
-// MP7 and MP9 have more room) of the smallest value, and the limiter moves
-// them only towards bounds that are at least 2 min - max.  Wavefronts all of
-// whose lanes are in that case skip the other two interface values.
+// limiter does.  The unlimited ones are at least (POS - CALM NEG) / DEN of the
+// smallest value, POS and NEG the sums of vor_plus's (and vor_minus's) positive
+// and negative weights: 0.76 for MP5, 0.70 for MP7, 0.65 for MP9, the higher
+// orders the tighter.  The limiter moves them only towards bounds that are at
+// least 2 min - max, (2 - CALM) of the smallest value: the tightest of all.
+// Wavefronts all of whose lanes are in that case skip the other two interface
+// values.
+template <int ORD> struct MPw;
+template <> struct MPw<5> { static constexpr int POS = 76, NEG = 16, DEN = 60; };
+template <> struct MPw<7> { static constexpr int POS = 562, NEG = 142, DEN = 420; };
+template <> struct MPw<9> { static constexpr int POS = 3512, NEG = 992, DEN = 2520; };
+constexpr double CALM = 1.9;
 template <int ORD, typename T> __device__ inline void mp_face_pos(const T* v, T& L, T& R) {
   constexpr int K = MPc<ORD>::K;
+  using W = MPw<ORD>;
+  static_assert(W::POS - W::NEG == W::DEN && W::POS > CALM * W::NEG && CALM < 2.0, "no negative value in the calm case");
   mp_face<ORD>(v, L, R);
   T lo = v[0], hi = v[0];
 #pragma unroll
@@ -294,7 +304,7 @@ template <int ORD, typename T> __device__ inline void mp_face_pos(const T* v, T&
     hi = lim_mx(hi, v[t]);
   }
   // a NaN stencil value is no fallback either way: L and R are NaN with it
-  if (__all(lo > T(0) && hi < T(1.9) * lo)) return;
+  if (__all(lo > T(0) && hi < T(CALM) * lo)) return;
   // cell i
   T up0 = L, um0 = mp_um<ORD>(v, K);
   T du0 = v[K] - v[K - 1], du1 = v[K + 1] - v[K];
