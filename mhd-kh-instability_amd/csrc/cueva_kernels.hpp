@@ -434,7 +434,7 @@ __global__ void k_stage_fused(Geom g, Planes P, Scheme S, int l, int halo, Statu
               P.p[P_PSI][ks], P.p[P_PHI][ks], P.p[P_Q][ks], out);
   store_stage(P.s, P.sf, k, out, l == 0, S.full != 0, false);
   if (P.kf[0])
-    store_kin(P.kf, k, P.p[P_VX][ks], P.p[P_VY][ks], P.p[P_VZ][ks], P.p[P_P][ks], P.p[P_RHO][ks], false);
+    store_kin(P.kf, k, P.p[P_VX][ks], P.p[P_VY][ks], P.p[P_VZ][ks], P.p[P_P][ks], P.p[P_RHO][ks]);
 }
 
 // Last stage right-hand side, sumfin, varfin and electricfield at one

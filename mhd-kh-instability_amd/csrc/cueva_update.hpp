@@ -282,8 +282,11 @@ __device__ inline void store_stage(double* const* s, float* const* sf, int64_t k
   if (sf[0]) store_stage<true>(s, sf, k, v, first, full, stream);
   else store_stage<false>(s, sf, k, v, first, full, stream);
 }
-__device__ inline void store_kin(float* const* kf, int64_t k, double vx, double vy, double vz, double p, double rho,
-                                 bool stream) {
+// The FP32 copies of the kinematics.  Like those of the stage state they are
+// stored through the caches on every grid: the next launch's stencils read
+// them, and streamed copies cost the learned recovery pass at 2048x4096 0.12 ms
+// (0.60 -> 0.72, before rows started cache lines).
+__device__ inline void store_kin(float* const* kf, int64_t k, double vx, double vy, double vz, double p, double rho) {
   static_assert(K_VX == 0 && K_VY == 1 && K_VZ == 2 && K_P == 3 && K_RHO == 4, "plane order");
   const double v[K_N] = {vx, vy, vz, p, rho};
   put_planes<K_N>(kf, k, v, false);
@@ -346,7 +349,7 @@ __device__ inline void recover_point(const Planes& P, const Scheme& S, const Sta
     stage_point(P, S, 0, k, false, o.vx, o.vy, o.vz, in.ex, in.ey, in.ez, in.bx, in.by, in.bz, o.rho, o.p,
                 nu[A_PSI], nu[A_PHI], nu[A_Q], sv);
     store_stage(P.sn, P.snf, k, sv, true, S.full != 0, S.stream > 0);
-    if (P.knf[0]) store_kin(P.knf, k, o.vx, o.vy, o.vz, o.p, o.rho, S.stream > 0);
+    if (P.knf[0]) store_kin(P.knf, k, o.vx, o.vy, o.vz, o.p, o.rho);
   }
 }
 
@@ -357,7 +360,7 @@ __device__ inline void stage0_after_c2p(Planes& P, const Scheme& S, int64_t k, c
   stage_point(P, S, 0, k, false, o.vx, o.vy, o.vz, in.ex, in.ey, in.ez, in.bx, in.by, in.bz, o.rho, o.p,
               P.p[P_PSI][k], P.p[P_PHI][k], P.p[P_Q][k], out);
   store_stage(P.s, P.sf, k, out, true, S.full != 0, S.stream > 1);
-  if (P.knf[0]) store_kin(P.knf, k, o.vx, o.vy, o.vz, o.p, o.rho, S.stream > 1);
+  if (P.knf[0]) store_kin(P.knf, k, o.vx, o.vy, o.vz, o.p, o.rho);
 }
 
 }  // namespace cueva
