@@ -154,6 +154,12 @@ int cueva_sync(cueva_ctx *ctx);
 int cueva_device_bytes(const cueva_ctx *ctx, int64_t *bytes);
 
 /* Host <-> device.  prims14 holds 14 planes of (imax+13)*(jmax+13) doubles.
+ * Host arrays go through pinned buffers that the ctx keeps from its first
+ * transfer until cueva_destroy, two of at most 4 MiB for each thread that
+ * copies; a transfer above 16 MiB takes up to 8 threads, the caller's among
+ * them and at most half of the CPUs the process may run on, which end with the
+ * call.  Without pinned memory, and for device memory given in place of a host
+ * array, strided copies do the same.
  * Upload replaces the RESTART read (03_restart_primitive.f95:50-61). */
 int cueva_upload_prims(cueva_ctx *ctx, const double *prims14);
 /* Download the 14 planes and, if cons5 != NULL, the evolved D tau Sx Sy Sz. */
@@ -294,7 +300,8 @@ int cueva_plane_range(cueva_ctx *ctx, int group, int index, double out[2]);
 
 /* Copy one device plane to the host (host layout).  group: 0 primitives
  * (14, restart order), 1 D tau Sx Sy Sz W, 2 stage planes, 3 x-face fluxes,
- * 4 y-face fluxes, 5+l stage-l right-hand sides (17).  For tests. */
+ * 4 y-face fluxes (3 and 4 as cueva_flux left them; cueva_step takes those
+ * planes as scratch), 5+l stage-l right-hand sides (17).  For tests. */
 int cueva_download_plane(cueva_ctx *ctx, int group, int index, double *out);
 
 /* Kernel timing on the ctx stream: while on, every launch is bracketed by

@@ -291,10 +291,12 @@ extern "C" int cueva_create(const cueva_params* p, cueva_ctx** out) {
   S.cm2 = 1.0;
   S.cm4 = (0.5 * ((1.0 - S.cm1) * (1.0 - S.cm1))) / S.cm1;
   imex_tables(p->order, p->mirk, S);
-  // by the bytes of a plane (a step touches about 70): the marching kernel's
-  // outputs from 4 MiB on (509x1021 gains 1.5 %, 300x700, 1.8 MB, loses 8 %), the
-  // recovery pass's, which has no stencil rows to keep, from 32 MiB on
-  // (2048x4096, 68 MB, gains 4 %, 1024x2048, 17 MB, loses 8 %)
+  // By the bytes of a plane (a step touches about 70).  Marching kernel from
+  // 4 MiB on; HLLC step with against without, FP64 / mixed, by MB a plane: 2.6
+  // +5 / +6 %, 6.6 -3 / -6, 10.7 -2 / -2, 17 -2 / -2, 26 -1 / -1, 47 -1 / 0, 68
+  // -1 / 0.  Recovery pass, which has no stencil rows to keep, from 32 MiB on:
+  // 10.7 +1 / -1 %, 17 0 / -1, 33 +0.3 / -1, 35 +0.4 / -1, 47 0 / -1, 68 -1 / -1:
+  // one line for both forms, at most 1 % from the better choice of either.
   const int64_t plane_bytes = g.plane * (int64_t)sizeof(double);
   S.stream = plane_bytes >= ((int64_t)32 << 20) ? 2 : plane_bytes >= ((int64_t)4 << 20) ? 1 : 0;
   c->rec_order = 5 + 2 * p->rec_mp;
@@ -313,10 +315,9 @@ extern "C" int cueva_create(const cueva_params* p, cueva_ctx** out) {
     e = getenv("CUEVA_MARCH_SEG");
     c->march_rows = e && atoi(e) > 0 ? atoi(e) : 0;
     // default off: inside the last marching launch the recovery's registers
-    // cost the whole launch occupancy or spill (FP32 faces at 2 waves per SIMD
-    // instead of 4; FP64 faces 256 B of scratch per lane): steps measured
-    // 0.83 ms (FP32 faces) and 0.12 ms (FP64 faces) slower at 2048x4096 than
-    // with the recovery in its own 0.55 ms pass
+    // spill at the launch's bound (HLLC: 54 VGPRs with FP64 faces, 122 with FP32
+    // ones): steps at 2048x4096 measured 5.15 against 4.99 ms (FP64 faces) and
+    // 3.56 against 3.29 (FP32 faces) with the recovery in its own 0.50 ms pass
     e = getenv("CUEVA_C2P_IN_MARCH");
     c->c2p_in_march = e ? atoi(e) != 0 : 0;
   }

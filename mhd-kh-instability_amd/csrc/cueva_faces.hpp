@@ -632,13 +632,15 @@ static_assert(offsetof(MarchArgs, P) == 0, "argument block layout");
 
 // Waves per SIMD the marching kernel is built for, a register bound (the
 // compiler spills past it).  Measured per step at 2048x4096:
-//   FP64: 2 for every solver.  HLLC fits 227 VGPRs, the MCL solvers 184-229;
-//     the others need a few more than 256 and ran 1 wave per SIMD unbounded:
-//     bounded, HLL runs 36 % faster, HLLE (one y-row buffer, below) 36 %,
-//     Lax-Friedrichs 32 %.  3 waves (168 VGPRs) spill 22-40 under HLLC and
-//     ran 12 % slower;
-//   FP32: 3.  With the stencils loaded ahead, 4 waves (128 VGPRs) spill
-//     and ran 3-6 % slower under HLLC, HLLE and HLL, 19 % under HLL + MC.
+//   FP64: 2 for every solver.  HLL, HLLE (with one y-row buffer, below) and
+//     HLLC take 219-222 VGPRs with MP5, 242-246 with MP9, the MCL solvers
+//     184-229: they fit 2 unbounded too (within 1 % of the same time).
+//     Lax-Friedrichs takes 266 unbounded, 1 wave per SIMD: 7.00 ms, bounded
+//     (12 spilled) 5.00.  3 waves (168 VGPRs) spill 22-40 under HLLC and ran
+//     12 % slower;
+//   FP32: 3 (144-162 VGPRs).  4 waves (128) spill 10-40: HLLC 3.42 against
+//     3.29 ms, HLL 3.50 / 3.24, HLL + MC 3.16 / 2.97, HLLE + MP7 at 1024x2048
+//     0.985 / 0.914.
 template <typename T, int SOLVER>
 constexpr int march_min_waves() {
   if constexpr (sizeof(T) == 8) return CUEVA_MARCH_F64_WAVES > 0 ? CUEVA_MARCH_F64_WAVES : 2;
@@ -656,8 +658,8 @@ constexpr int march_y_buffers() {
 
 // Wavefronts per block = face rows per tile step: 4.  More re-read fewer halo
 // rows (a tile step reads MW + 5), but the barriers then wait for more of
-// them: HLLC + MP5 at 2048x4096 with 4 / 6 / 8 waves, FP64 5.12 / 6.45 / 5.49
-// ms per step, FP32 4.15 / 4.93 / 4.53 (12 waves 4.30).
+// them: HLLC + MP5 at 2048x4096 with 4 / 6 / 8 waves, FP64 4.99 / 6.24 / 5.41
+// ms per step, FP32 3.29 / 4.01 / 3.57.
 #ifndef CUEVA_MARCH_F32_BLOCK_WAVES
 #define CUEVA_MARCH_F32_BLOCK_WAVES 4
 #endif

@@ -46,8 +46,8 @@ __device__ inline void copy_ghosts(ST* const* a, int n, int nzero, int k0, int64
 // One thread copies one ghost point of GHOST_PLANES planes (blockIdx.y picks
 // them), their loads in flight together.  The fill is bound by latency: a
 // thread that walked all the planes had one load and one store in flight at a
-// time and took 14 us at 32x64, 21 at 128x256 and 36 at 2048x4096; now
-// 6.5, 6.6 and 21 us.  The bands left and right are walked row by row, 12
+// time and took 14 us between events at 32x64, 21 at 128x256 and 36 at
+// 2048x4096; now 6.5, 6.5 and 15.5 us (mixed, with its FP32 copies, 18.5).  The bands left and right are walked row by row, 12
 // points each, so that neighbouring threads share cache lines.
 __global__ void __launch_bounds__(256) k_fill_ghosts(Geom g, PlaneList pl, StatusRef sr) {
   if (halted(sr)) return;

@@ -13,12 +13,11 @@ struct Rhs { double r[R_N]; };
 // Values that no later part of the launch reads, n planes at offset k.  On
 // large grids they are stored past the caches (non-temporal, Scheme::stream):
 // the marching kernel's 34 output planes a cell otherwise push out the stencil
-// rows that its next tile step reads again.  With against without, at
-// 2048x4096: fabric traffic of an FP32 stage launch 7.3 against 7.9 GB, step
-// FP64 HLLC 5.07 against 5.13 ms, mixed HLL 3.98 against 4.09; mixed HLLE + MP7
-// at 1024x2048 1.20 against 1.24.  Small grids, whose planes the 256 MB
-// Infinity Cache keeps from launch to launch, lose by it (HLL + MC at 300x700
-// 201 against 186 us).
+// rows that its next tile step reads again.  With against without, both
+// passes: 2048x4096 step FP64 HLLC 4.95 against 5.04 ms, mixed HLL 3.22 against
+// 3.28; marching only, mixed HLLC at 620x1240 0.351 against 0.372.  Small grids,
+// whose planes the 256 MB Infinity Cache keeps from launch to launch, lose by it
+// (FP64 HLLC at 380x760 232 against 221 us).
 template <int N, typename ST>
 __device__ inline void put_planes(ST* const* p, int64_t k, const double* v, bool stream) {
   if (stream) {
